@@ -948,18 +948,25 @@ int short_run_launch(const AttnArgs& a, int groups, int pps, hipStream_t s) {
 // blocks lose (8.84 us at 1 sequence).
 constexpr int kTwoWavePairs = 8;
 
+// Whether a call in kv groups of the given number takes the short-run grid: its splits are at most
+// kShortRunPages pages long and its (sequence, kv group) pairs at most kSplitGridPairs.
+bool short_runs(const AttnArgs& a, int groups) {
+  const int pps = (a.max_pages + a.num_splits - 1) / a.num_splits;
+  return a.part_o && a.num_splits >= 3 && pps <= kShortRunPages &&
+         (long long)a.n_seq * groups <= kSplitGridPairs;
+}
+
 template <int KVW>
 int attn_launch(const AttnArgs& a, hipStream_t s) {
   const int groups = KVW == 8 ? (a.n_kv_heads + 7) / 8 : a.n_kv_heads / KVW;
   const int pps = (a.max_pages + a.num_splits - 1) / a.num_splits;  // pages per split
-  const bool short_runs = a.part_o && a.num_splits >= 3 && pps <= kShortRunPages &&
-                          (long long)a.n_seq * groups <= kSplitGridPairs;
+  const bool short_run = short_runs(a, groups);
   // The page-balanced kernel counts the batch's units in 32-bit ints: at most
   // n_seq * (start_units + max_pages) of them. Batches that could exceed that take the
   // sequence-split grid, which needs no count.
   const bool units_fit =
       (long long)a.n_seq * (start_units<KVW>() + (long long)a.max_pages) <= 0x7FFFFFFFLL;
-  if (a.num_splits >= 3 && a.part_o && !short_runs && units_fit) {
+  if (a.num_splits >= 3 && a.part_o && !short_run && units_fit) {
     int blocks = balanced_blocks() / groups;
     if (blocks < 1) blocks = 1;
     int st = launch(k_attn_balanced<KVW>, dim3((unsigned)blocks, (unsigned)groups), dim3(kThreads),
@@ -971,7 +978,7 @@ int attn_launch(const AttnArgs& a, hipStream_t s) {
                   a.max_pages, a.n_heads, a.num_splits, 0);
   }
   int st;
-  if (short_runs) {
+  if (short_run) {
     if constexpr (KVW == 2) {
       st = (long long)a.n_seq * groups <= kTwoWavePairs
                ? short_run_launch<KVW, 2>(a, groups, pps, s)
@@ -983,7 +990,7 @@ int attn_launch(const AttnArgs& a, hipStream_t s) {
     st = split_launch<KVW, 0, false>(a, groups, pps, s);
   }
   if (st != 0 || pps >= a.max_pages) return st;  // every sequence fits in one split
-  if (short_runs) {
+  if (short_run) {
     const dim3 mgrid((unsigned)a.n_heads, (unsigned)a.n_seq);
     return launch(k_attn_merge_many, mgrid, dim3(64), 0, s, a.part_o, a.part_ml, a.lens, a.out,
                   a.max_pages, a.n_heads, a.num_splits, pps);
@@ -1027,7 +1034,8 @@ static int check_attention(const uint16_t* q, const uint16_t* k_pool, const uint
   return -1;
 }
 
-// Kv heads per kv group (one grid row of blocks each). Rows of 1, 2 or 4 kv heads put several
+// Kv heads per kv group (one grid row of blocks each) for the short-run grid and for calls of one
+// or two splits. Rows of 1, 2 or 4 kv heads put several
 // positions in one row read. Any other count takes groups of 8 (the last one partly idle when
 // the count is not a multiple of 8), except for very small batches. At most 8 (sequence, kv
 // group) pairs cut their rows into narrower groups: 4 or 2 heads of 2 or 4 positions per row
@@ -1035,7 +1043,7 @@ static int check_attention(const uint16_t* q, const uint16_t* k_pool, const uint
 // positions, 8 kv heads: 1 sequence 10.31 -> 8.25 us with groups of 2, 2 sequences 10.44 ->
 // 8.71, 4 sequences 10.67 -> 9.67 with groups of 4. At 8 or more sequences, groups of 8 are as
 // fast or faster; groups of 1 lose everywhere.
-static int kv_group_width(int n_seq, int n_kv_heads) {
+static int short_run_width(int n_seq, int n_kv_heads) {
   if (n_kv_heads == 1 || n_kv_heads == 2 || n_kv_heads == 4) {
     int w = n_kv_heads;
     while (w > 2 && (long long)n_seq * (n_kv_heads / (w / 2)) <= 8) w /= 2;
@@ -1043,6 +1051,25 @@ static int kv_group_width(int n_seq, int n_kv_heads) {
   }
   for (int w = 2; w <= 4; w *= 2)  // the narrowest width whose pairs fit
     if (n_kv_heads % w == 0 && (long long)n_seq * (n_kv_heads / w) <= 8) return w;
+  return 8;
+}
+
+// Kv heads per kv group for the page-balanced grid, which every call takes that the short-run
+// grid does not. A sequence has at most num_splits - 1 segments per kv group, so a few long
+// sequences cannot fill 256 CUs in groups of 8 heads: 5 sequences of up to 16384 positions (1024
+// pages, runs of at least ceil(1023 / 30) = 35) leave 115 blocks, each reading 35 pages one
+// after the other. Narrower groups cut the same pages into more, shorter runs; past the counts
+// below the narrower row reads (KVW * 128 contiguous bytes per position) and the second and third
+// scan of the lengths cost more than the balance gains. Same box, 8 kv heads, both kernels, us, in
+// groups of 8 / 4 / 2: 1 x 16384 42.8 / 28.1 / 20.8, 5 x U[1, 16384] 43.2 / 29.7 / 28.3,
+// 8 x U[1, 4096] 21.1 / 17.1 / 16.0, 12 x U[1, 8192] 29.9 / 28.4 / 28.2, 16 x U[1, 8192]
+// 32.6 / 31.0 / 31.6, 24 x U[1, 2048] 18.9 / 17.2 / 17.8, 64 x U[1, 4096] 47.8 / 46.1 / 48.0,
+// 96 x U[1, 2048] 39.7 / 39.8 / 41.5, 128 x U[1, 512] 19.7 / 20.3 / 24.5, 256 x U[1, 2048]
+// 93.7 / 95.2 / 96.2.
+static int balanced_width(int n_seq, int n_kv_heads) {
+  if (n_kv_heads % 2 == 0 && (long long)n_seq * (n_kv_heads / 2) <= 48) return 2;
+  if (n_kv_heads % 4 == 0 && (long long)n_seq * (n_kv_heads / 4) <= 128) return 4;
+  if (n_kv_heads == 1 || n_kv_heads == 2 || n_kv_heads == 4) return n_kv_heads;
   return 8;
 }
 
@@ -1067,7 +1094,10 @@ static int run_attention(const uint16_t* q, const uint16_t* k_pool, const uint16
   a.n_kv_heads = n_kv_heads;
   a.num_splits = num_splits;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  switch (kv_group_width(n_seq, n_kv_heads)) {
+  int width = short_run_width(n_seq, n_kv_heads);
+  if (a.part_o && num_splits >= 3 && !short_runs(a, (n_kv_heads + width - 1) / width))
+    width = balanced_width(n_seq, n_kv_heads);
+  switch (width) {
     case 4: return attn_launch<4>(a, s);
     case 2: return attn_launch<2>(a, s);
     case 1: return attn_launch<1>(a, s);

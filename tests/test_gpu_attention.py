@@ -140,6 +140,29 @@ def test_very_small_batches_take_narrower_kv_groups(llmk, orc, lens, nkv):
                    f"lens {lens} n_kv {nkv} splits {splits}")
 
 
+@pytest.mark.parametrize("n_seq,nkv", [(1, 8), (12, 8), (13, 8), (64, 8), (65, 8), (16, 6),
+                                       (17, 6), (32, 16), (33, 16), (25, 4), (10, 12)])
+def test_page_balanced_grid_narrows_its_kv_groups_for_few_sequences(llmk, orc, n_seq, nkv):
+    """The page-balanced grid takes groups of 2 heads up to 48 (sequence, group) pairs, of 4 up to
+    128 and of 8 beyond: both sides of each line, with one sequence long enough that the split
+    count bounds its runs (3 splits leave two segments) and others of one position or none."""
+    rng = np.random.default_rng(500 + 17 * n_seq + nkv)
+    lens = rng.integers(1, 200, n_seq)
+    lens[n_seq // 2] = 1700
+    lens[-1] = 1 if n_seq < 3 else 0
+    if n_seq == 1:
+        lens[0] = 2100
+    c = attention_case(rng, tuple(int(x) for x in lens), n_heads=4 * nkv, n_kv_heads=nkv)
+    d = OnDevice(c)
+    ref = oracle_out(orc, c).reshape(n_seq, -1)
+    some = lens > 0
+    for splits in (3, 20):
+        got = d.run(llmk, splits).reshape(n_seq, -1)
+        assert_tol(orc.compare(got[some].reshape(-1), ref[some].reshape(-1)), EXACT_FLOOR,
+                   f"{n_seq} sequences n_kv {nkv} splits {splits}")
+        assert np.isnan(got[~some].view(np.float16)).all()
+
+
 @pytest.mark.parametrize("n_seq", [1024, 1025, 3000])
 def test_many_sequences(llmk, orc, n_seq):
     """Batches around and past the 1024 sequences (4 tiles of 256 threads) whose page counts the
