@@ -30,6 +30,7 @@
 
 #include <mutex>
 
+#include "attention.hpp"
 #include "common.hpp"
 
 namespace llmk {
@@ -1001,6 +1002,17 @@ int attn_launch(const AttnArgs& a, hipStream_t s) {
 }
 
 }  // namespace
+
+int merge_split_pieces(const float* workspace, const int32_t* lens, uint16_t* out, int n_rows,
+                       int max_pages, int n_heads, int num_splits, int pages_per_split,
+                       hipStream_t stream) {
+  const float2* ml = reinterpret_cast<const float2*>(
+      workspace + (size_t)n_rows * num_splits * n_heads * kHeadDim);
+  return launch(k_attn_merge, dim3((unsigned)((n_heads + 7) / 8), (unsigned)n_rows), dim3(64), 0,
+                stream, workspace, ml, lens, reinterpret_cast<f16*>(out), max_pages, n_heads,
+                num_splits, pages_per_split);
+}
+
 }  // namespace llmk
 
 using namespace llmk;

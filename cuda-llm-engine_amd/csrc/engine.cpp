@@ -42,6 +42,7 @@
 #include <unordered_map>
 #include <vector>
 
+#include "attention.hpp"
 #include "llmk.h"
 
 namespace {
@@ -80,6 +81,10 @@ struct llmk_engine {
   hipEvent_t staged = nullptr;
   int32_t *tokens = nullptr, *positions = nullptr, *lens = nullptr, *logit_rows = nullptr,
           *tables = nullptr;
+  // The pass's prompt rows (see find_tiles): the tiles, and the lengths of the rows in none
+  // (0 in the others) and of the rows in one.
+  llmk::PromptTile* tiles = nullptr;
+  int32_t *row_lens = nullptr, *tile_lens = nullptr;
 
   // activations (one allocation)
   void* act_buf = nullptr;
@@ -91,17 +96,22 @@ struct llmk_engine {
 
   // Pages the longest attention of the rows last set reads (position / 16 + 1).
   int rows_span = 0;
+  // The tiles of the rows last set, the pages the longest attention of their rows reads, and the
+  // rows in none.
+  int n_tiles = 0, tile_span = 0, loose_rows = 0;
+  long long tile_positions = 0;  // positions that the tiles' rows attend to, summed over the rows
   // Rows and logit rows uploaded by the last llmk_engine_set_rows: a pass may not ask for more,
   // since the device copies past them hold no checked indices.
   int rows_set = 0, logit_rows_set = 0;
 
   // HIP graphs of the forward pass, keyed by (n_rows, n_logit_rows, resolved num_splits,
-  // host_argmax: whether the pass ends before the GPU argmax)
+  // host_argmax: whether the pass ends before the GPU argmax, n_tiles, tile_span and whether rows
+  // are left over, the last three 0 for a pass that takes no tiles)
   struct Graph {
     bool seen = false;
     hipGraphExec_t exec = nullptr;
   };
-  std::map<std::tuple<int, int, int, int>, Graph> graphs;
+  std::map<std::tuple<int, int, int, int, int, int, int>, Graph> graphs;
   hipStream_t sched_stream = nullptr;  // the stream the scheduler callbacks run on
   bool fuse_rows = true;  // passes of <= LLMK_LINEAR_ROWS_MAX rows use the fused projections
   // LLMK_ENGINE_HOST_ARGMAX: the pass ends with the logits; the scheduler callbacks copy them
@@ -161,6 +171,50 @@ void carve_inputs(llmk_engine* e, Carver& c) {
   e->lens = c.take<int32_t>(R);
   e->logit_rows = c.take<int32_t>(R);
   e->tables = c.take<int32_t>(R * e->max_pages);
+  e->row_lens = c.take<int32_t>(R);
+  e->tile_lens = c.take<int32_t>(R);
+  e->tiles = c.take<llmk::PromptTile>(R);
+}
+
+// Rows of one sequence from which consecutive positions form tiles: below, the rows run as decode
+// rows (a pass of up to LLMK_LINEAR_ROWS_MAX rows has none). From 9 rows up tiles are as fast or
+// faster: two layers, us, 9 rows from position 1024 180 -> 176, from 0 equal, 33 from 1024
+// 205 -> 188.
+constexpr int kTileMinRows = 9;
+
+// Finds the runs of rows that continue one another: positions ascending by one, block tables
+// equal on every page the later row reads. Each run of at least kTileMinRows rows is cut into
+// tiles of kTileRows; fills tiles, row_lens and tile_lens and returns the tile count. The caller
+// has checked every position and table entry.
+int find_tiles(int n, const int32_t* positions, const int32_t* tables, int max_pages,
+               llmk::PromptTile* tiles, int32_t* row_lens, int32_t* tile_lens, int* span,
+               int* loose, long long* attended) {
+  int count = 0;
+  *span = *loose = 0;
+  *attended = 0;
+  for (int r = 0; r < n;) {
+    int end = r + 1;
+    while (end < n && positions[end] == positions[end - 1] + 1 &&
+           memcmp(tables + (size_t)(end - 1) * max_pages, tables + (size_t)end * max_pages,
+                  (size_t)(positions[end - 1] / kPage + 1) * sizeof(int32_t)) == 0)
+      ++end;
+    const bool tiled = end - r >= kTileMinRows;
+    for (int i = r; i < end; ++i) {
+      row_lens[i] = tiled ? 0 : positions[i] + 1;
+      tile_lens[i] = tiled ? positions[i] + 1 : 0;
+      *attended += tile_lens[i];
+    }
+    if (tiled) {
+      for (int i = r; i < end; i += llmk::kTileRows)
+        tiles[count++] = {i, end - i < llmk::kTileRows ? end - i : llmk::kTileRows};
+      const int pages = positions[end - 1] / kPage + 1;
+      *span = pages > *span ? pages : *span;
+    } else {
+      *loose += end - r;
+    }
+    r = end;
+  }
+  return count;
 }
 
 void carve_activations(llmk_engine* e, Carver& c) {
@@ -429,6 +483,9 @@ extern "C" int llmk_engine_set_rows(llmk_engine* e, int n_rows, const int32_t* t
   int32_t* h_lens = c.take<int32_t>(e->max_rows);
   int32_t* h_logit = c.take<int32_t>(e->max_rows);
   int32_t* h_tables = c.take<int32_t>((size_t)e->max_rows * P);
+  int32_t* h_row_lens = c.take<int32_t>(e->max_rows);
+  int32_t* h_tile_lens = c.take<int32_t>(e->max_rows);
+  llmk::PromptTile* h_tiles = c.take<llmk::PromptTile>(e->max_rows);
   memcpy(h_tokens, tokens, n_rows * sizeof(int32_t));
   memcpy(h_pos, positions, n_rows * sizeof(int32_t));
   int span = 0;
@@ -439,6 +496,8 @@ extern "C" int llmk_engine_set_rows(llmk_engine* e, int n_rows, const int32_t* t
   e->rows_span = span;
   if (n_logit_rows > 0) memcpy(h_logit, logit_rows, n_logit_rows * sizeof(int32_t));
   memcpy(h_tables, block_tables, (size_t)n_rows * P * sizeof(int32_t));
+  e->n_tiles = find_tiles(n_rows, positions, block_tables, P, h_tiles, h_row_lens, h_tile_lens,
+                          &e->tile_span, &e->loose_rows, &e->tile_positions);
   hipStream_t s = static_cast<hipStream_t>(stream);
   st = (int)hipMemcpyAsync(e->in_buf, e->staging, e->in_bytes, hipMemcpyHostToDevice, s);
   if (st == LLMK_OK) st = (int)hipEventRecord(e->staged, s);
@@ -478,6 +537,52 @@ static int resolve_splits(const llmk_engine* e, int n, int num_splits, bool capt
     if (num_splits < 1) num_splits = 1;
   }
   return num_splits > kMaxSplits ? kMaxSplits : num_splits;
+}
+
+// Passes that mix decode rows with prompt rows attending to fewer positions in all than this run
+// them all as decode rows: the tiles' launch, and their merge where they are split, come on top of
+// the decode rows' two. Two layers, us, as decode rows -> in tiles: 10 sequences and 256 rows from
+// position 0 (33 thousand positions) 312 -> 328, 32 and 300 (45 thousand) 338 -> 347, 20 and 100
+// from position 500 (55 thousand) 259 -> 264, 20 and 400 from there (280 thousand) 456 -> 364.
+constexpr long long kMixedMinPositions = 81920;
+
+// Whether a pass over n rows runs its prompt rows in tiles: the rows last set, all of them, hold
+// some, and the pass is not being captured by the caller (its replays run rows set later, which
+// may hold others).
+static bool takes_tiles(const llmk_engine* e, int n, bool capturing) {
+  return !capturing && e->n_tiles > 0 && n == e->rows_set &&
+         (e->loose_rows == 0 || e->tile_positions >= kMixedMinPositions);
+}
+
+// Attention of layer l over the pass's rows: prompt tiles share the K and V rows they read
+// (attention_prompt.hip); the other rows, or all of them without tiles, are decode rows. The
+// decode launch comes first: it writes NaN to rows of length 0, those in a tile.
+static int attention(llmk_engine* e, int l, int n, bool tiled, int num_splits, void* s) {
+  const llmk_model_config& m = e->cfg;
+  if (!tiled || e->loose_rows > 0) {
+    const int st = llmk_attention_decode_fast(
+        e->q, e->k_pool[l], e->v_pool[l], e->tables, tiled ? e->row_lens : e->lens, e->attn, e->ws,
+        n, e->max_pages, kPage, m.n_heads, m.n_kv_heads, m.head_dim, num_splits, s);
+    if (st != LLMK_OK || !tiled) return st;
+  }
+  llmk::PromptAttention a;
+  a.q = e->q;
+  a.k_pool = e->k_pool[l];
+  a.v_pool = e->v_pool[l];
+  a.tables = e->tables;
+  a.positions = e->positions;
+  a.lens = e->tile_lens;
+  a.tiles = e->tiles;
+  a.out = e->attn;
+  a.workspace = e->ws;
+  a.n_rows = n;
+  a.n_tiles = e->n_tiles;
+  a.max_pages = e->max_pages;
+  a.n_heads = m.n_heads;
+  a.n_kv_heads = m.n_kv_heads;
+  llmk::prompt_splits(e->n_tiles, m.n_kv_heads, e->tile_span, kMaxSplits, &a.num_splits,
+                      &a.pages_per_split);
+  return llmk::prompt_attention(a, static_cast<hipStream_t>(s));
 }
 
 // Whether a pass over n rows takes the fused few-rows path: every projection is a
@@ -566,25 +671,13 @@ extern "C" int llmk_engine_set_option(llmk_engine* e, int option, int value) {
   }
 }
 
-extern "C" int llmk_engine_forward(llmk_engine* e, int n_rows, int n_logit_rows, int num_splits,
-                                   void* stream) {
-  if (!e || n_rows < 0 || n_rows > e->max_rows || n_logit_rows > n_rows)
-    return LLMK_ERR_INVALID_VALUE;
-  if (n_rows == 0) return LLMK_OK;
-  if (!rows_uploaded(e, n_rows, n_logit_rows)) return LLMK_ERR_INVALID_VALUE;
+// The pass of llmk_engine_forward, its arguments checked and num_splits resolved.
+static int forward_pass(llmk_engine* e, int n, int n_logit_rows, int num_splits, bool tiled,
+                        void* s) {
   const llmk_model_config& m = e->cfg;
-  const int n = n_rows, H = m.hidden, L = m.n_layers;
+  const int H = m.hidden, L = m.n_layers;
   const bool all_rows = n_logit_rows < 0;
   const int nl = all_rows ? n : n_logit_rows;
-  bool capturing = false;
-  if (num_splits <= 0) {
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    const int st = (int)hipStreamIsCapturing(static_cast<hipStream_t>(stream), &cap);
-    if (st != LLMK_OK) return st;
-    capturing = cap != hipStreamCaptureStatusNone;
-  }
-  num_splits = resolve_splits(e, n, num_splits, capturing);
-  void* s = stream;
   if (fused_rows_path(e, n)) return forward_fused_rows(e, n, nl, all_rows, num_splits, s);
 #define LLMK_TRY(call)               \
   do {                               \
@@ -599,9 +692,7 @@ extern "C" int llmk_engine_forward(llmk_engine* e, int n_rows, int n_logit_rows,
     LLMK_TRY(llmk_qkv_rope_scatter(e->qkv, e->qkvdim, e->q, e->k_pool[l], e->v_pool[l],
                                    e->tables, e->positions, e->inv_freq, n, e->max_pages, kPage,
                                    m.n_heads, m.n_kv_heads, m.head_dim, s));
-    LLMK_TRY(llmk_attention_decode_fast(e->q, e->k_pool[l], e->v_pool[l], e->tables, e->lens,
-                                        e->attn, e->ws, n, e->max_pages, kPage, m.n_heads,
-                                        m.n_kv_heads, m.head_dim, num_splits, s));
+    LLMK_TRY(attention(e, l, n, tiled, num_splits, s));
     LLMK_TRY(llmk_linear(e->blas, e->attn, w.wo, e->proj, n, e->qdim, H, s));
     LLMK_TRY(llmk_add_rmsnorm(e->x, e->proj, w.mlp_norm, e->normed, n, H, m.eps, s));
     LLMK_TRY(llmk_linear(e->blas, e->normed, w.wgu, e->gu, n, H, 2 * m.inter, s));
@@ -629,6 +720,23 @@ extern "C" int llmk_engine_forward(llmk_engine* e, int n_rows, int n_logit_rows,
   if (!e->host_argmax) LLMK_TRY(llmk_argmax_rows(e->logits, e->next, nl, m.vocab, s));
 #undef LLMK_TRY
   return LLMK_OK;
+}
+
+extern "C" int llmk_engine_forward(llmk_engine* e, int n_rows, int n_logit_rows, int num_splits,
+                                   void* stream) {
+  if (!e || n_rows < 0 || n_rows > e->max_rows || n_logit_rows > n_rows)
+    return LLMK_ERR_INVALID_VALUE;
+  if (n_rows == 0) return LLMK_OK;
+  if (!rows_uploaded(e, n_rows, n_logit_rows)) return LLMK_ERR_INVALID_VALUE;
+  bool capturing = false;
+  if (num_splits <= 0 || e->n_tiles > 0) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    const int st = (int)hipStreamIsCapturing(static_cast<hipStream_t>(stream), &cap);
+    if (st != LLMK_OK) return st;
+    capturing = cap != hipStreamCaptureStatusNone;
+  }
+  return forward_pass(e, n_rows, n_logit_rows, resolve_splits(e, n_rows, num_splits, capturing),
+                      takes_tiles(e, n_rows, capturing), stream);
 }
 
 extern "C" void* llmk_engine_buffer(llmk_engine* e, int which, int layer) {
@@ -663,16 +771,18 @@ extern "C" int llmk_engine_forward_graph(llmk_engine* e, int n_rows, int n_logit
   if (n_rows == 0) return LLMK_OK;
   if (!rows_uploaded(e, n_rows, n_logit_rows)) return LLMK_ERR_INVALID_VALUE;
   num_splits = resolve_splits(e, n_rows, num_splits);  // the key holds the launch shapes
-  llmk_engine::Graph& g = e->graphs[std::make_tuple(n_rows, n_logit_rows < 0 ? -1 : n_logit_rows,
-                                                    num_splits, e->host_argmax ? 1 : 0)];
+  const bool tiled = takes_tiles(e, n_rows, false);
+  llmk_engine::Graph& g = e->graphs[std::make_tuple(
+      n_rows, n_logit_rows < 0 ? -1 : n_logit_rows, num_splits, e->host_argmax ? 1 : 0,
+      tiled ? e->n_tiles : 0, tiled ? e->tile_span : 0, tiled && e->loose_rows > 0 ? 1 : 0)];
   if (g.exec) return (int)hipGraphLaunch(g.exec, s);
   if (!g.seen) {  // first use: eager, which also makes the GEMM plans of these shapes
     g.seen = true;
-    return llmk_engine_forward(e, n_rows, n_logit_rows, num_splits, stream);
+    return forward_pass(e, n_rows, n_logit_rows, num_splits, tiled, stream);
   }
   st = (int)hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal);
   if (st != LLMK_OK) return st;
-  const int fwd = llmk_engine_forward(e, n_rows, n_logit_rows, num_splits, stream);
+  const int fwd = forward_pass(e, n_rows, n_logit_rows, num_splits, tiled, stream);
   hipGraph_t graph = nullptr;
   st = (int)hipStreamEndCapture(s, &graph);
   if (fwd != LLMK_OK || st != LLMK_OK) {

@@ -444,7 +444,11 @@ LLMK_API int llmk_engine_set_rows(llmk_engine* e, int n_rows, const int32_t* tok
  * pages (no merge launch), else LLMK_ATTN_TARGET_BLOCKS / (n_rows * n_kv_heads) at most
  * max_pages; always capped at 32, the workspace. On a stream that is being captured the first
  * rule is skipped, so that a captured pass keeps enough splits for the longer contexts it may
- * be replayed with. Allocates nothing; capturable into a HIP graph for a fixed n_rows.
+ * be replayed with. Runs of 9 or more rows that continue one another (consecutive positions of
+ * one sequence: a prompt) attend in tiles that share the K and V rows they read, when n_rows is
+ * all the rows last set; not on a stream being captured, whose replays may hold other rows. Either
+ * way gives the same values up to fp32 rounding. Allocates nothing; capturable into a HIP graph
+ * for a fixed n_rows.
  * ref: engine/batched.cu:107-120 (decode_step_gpu), :44-72 (layer_forward_batched), :150
  * (argmax_rows in model_decode_batch_greedy). */
 LLMK_API int llmk_engine_forward(llmk_engine* e, int n_rows, int n_logit_rows, int num_splits,

@@ -593,6 +593,117 @@ def test_engine_graph_replays_match_eager(llmk, orc):
         assert torch.equal(e.pool(llmk.BUF_K_POOL, 1).view(torch.int16), ref_pool), f"replay {r}"
 
 
+def run_both_ways(llmk, e, rows, logit_rows, fill):
+    """The rows eagerly (prompt rows in tiles) and captured by the caller (every row a decode
+    row): (logits, residual, K pool, V pool of the last layer) of each."""
+    n, nl, out = len(rows[0]), len(logit_rows), []
+    stream = torch.cuda.Stream()
+    for captured in (False, True):
+        for l in range(e.cfg.n_layers):
+            for which in (llmk.BUF_K_POOL, llmk.BUF_V_POOL):
+                e.write_pool(which, l, fill)
+        e.set_rows(*rows, logit_rows)
+        if captured:
+            g = torch.cuda.CUDAGraph()
+            torch.cuda.synchronize()
+            with torch.cuda.graph(g, stream=stream):
+                e.forward(n, nl, stream=stream)
+            g.replay()
+        else:
+            e.forward(n, nl)
+        torch.cuda.synchronize()
+        out.append((e.logits(nl), e.residual(n), e.pool(llmk.BUF_K_POOL, e.cfg.n_layers - 1),
+                    e.pool(llmk.BUF_V_POOL, e.cfg.n_layers - 1)))
+    return out
+
+
+# (length, start) of each prompt and the position of each decode row, in the order of the rows
+PROMPT_PASSES = [
+    [(9, 0)], [(31, 0)], [(32, 1)], [(33, 0)], [(64, 15)], [(65, 16)], [(130, 100)],
+    [(10, 250)],                             # few rows far into a sequence: split over positions
+    [(16, 5), (8, 40), (40, 0)],             # 8 rows are too few for a tile
+    [0, 77, (20, 30), 5, (45, 0), 130, 131],  # decode rows around and between the prompts
+]
+
+
+@pytest.mark.parametrize("odd", [False, True], ids=["finite", "infinite_v"])
+@pytest.mark.parametrize("parts", PROMPT_PASSES, ids=[str(i) for i in range(len(PROMPT_PASSES))])
+def test_prompt_tiles_match_decode_rows(llmk, parts, odd):
+    """A pass's prompt rows in tiles against the same rows as decode rows, at the edges of tiles,
+    chunks of 64 positions and pages; every slot past a sequence's end holds NaN. With odd, the
+    second layer's V has infinite elements in about a quarter of the new positions: a row that
+    sees none stays finite, and the others have NaN where the decode rows have it. Both ways
+    round one fp16 result per element from fp32 sums, so after two layers they differ by fp16
+    roundings (2^-11 each, a few of them in a chain)."""
+    cfg = dict(TINY, n_heads=8, n_kv_heads=2)
+    w = tiny_weights(0x5EED0260, embed_std=0.5, cfg=cfg)
+    if odd:
+        name = "model.layers.1.self_attn.v_proj.weight"
+        v = np.array(w[name].view(np.float16))
+        v[0, :] = 0.0
+        v[0, 0] = 60000.0
+        w[name] = v.view(w[name].dtype)
+    rng = np.random.default_rng(0x5EED0261)
+    max_pages = 18
+    tables = rng.permutation(len(parts) * max_pages).astype(np.int32).reshape(-1, max_pages)
+    tok, pos, tab, last = [], [], [], []
+    ends = []
+    for t, part in zip(tables, parts):
+        n, start = part if isinstance(part, tuple) else (1, part)
+        pos += range(start, start + n)
+        tab += [t] * n
+        last.append(len(pos) - 1)
+        ends.append(start + n)
+    tok = rng.integers(0, cfg["vocab"], len(pos)).astype(np.int32)
+    kvdim = 64 * cfg["n_kv_heads"]
+    fill = torch.full((tables.size * 16, kvdim), float("nan"), dtype=torch.float16)
+    for t, end in zip(tables, ends):
+        for p in range(end):
+            fill[t[p // 16] * 16 + p % 16] = torch.from_numpy(
+                rng.standard_normal(kvdim).astype(np.float16))
+    e = make_engine(llmk, cfg, w, len(pos), max_pages, int(tables.size))
+    rows = (tok, np.array(pos, np.int32), np.array(tab, np.int32))
+    got, ref = run_both_ways(llmk, e, rows, last, fill)
+    seen_nan = False
+    for name, a, b in zip(("logits", "residual", "k", "v"), got, ref):
+        a, b = a.double(), b.double()
+        assert torch.equal(torch.isnan(a), torch.isnan(b)), name
+        fin = torch.isfinite(b)
+        assert torch.equal(a[~fin].nan_to_num(), b[~fin].nan_to_num()), name
+        if name in ("logits", "residual"):
+            seen_nan = seen_nan or not bool(fin.all())
+            assert bool(fin.any()) or odd
+        d = a[fin] - b[fin]
+        assert d.norm() <= 2e-3 * max(float(b[fin].norm()), 1e-6), (name, float(d.norm()))
+    assert seen_nan == odd or len(pos) < 12
+
+
+def test_prompt_tiles_replayed_with_other_rows(llmk):
+    """The engine's own graph of a pass with prompt rows, replayed after other rows of the same
+    counts were set: each replay gives the bits of an eager pass over its rows."""
+    w = tiny_weights(0x5EED0270, embed_std=0.5)
+    rng = np.random.default_rng(0x5EED0271)
+    e = make_engine(llmk, TINY, w, 64, 8, 32)
+    s = torch.cuda.Stream()
+    for rep in range(4):
+        table = rng.permutation(32).astype(np.int32)[:8]
+        n = 40
+        rows = (rng.integers(0, TINY["vocab"], n).astype(np.int32),
+                np.arange(60, 60 + n, dtype=np.int32), np.array([table] * n))
+        fill = torch.from_numpy(rng.standard_normal(32 * 16 * 64).astype(np.float16))
+        out = []
+        for graph in (False, True):
+            for l in range(e.cfg.n_layers):
+                e.write_pool(llmk.BUF_K_POOL, l, fill)
+                e.write_pool(llmk.BUF_V_POOL, l, fill)
+            torch.cuda.synchronize()
+            e.set_rows(*rows, [n - 1], stream=s)
+            (e.forward_graph if graph else e.forward)(n, 1, stream=s)
+            torch.cuda.synchronize()
+            out.append((e.logits(1).view(torch.int16), e.residual(n).view(torch.int16)))
+        assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1]), rep
+
+
 def test_engine_loads_the_reference_weight_format(llmk, tmp_path):
     weights = importlib.import_module("llmk.weights")
     w = tiny_weights(0x5EED0250, embed_std=0.5)
