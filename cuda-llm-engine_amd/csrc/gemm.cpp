@@ -2,8 +2,9 @@
 // PyTorch Linear without bias), fp16 in and out, fp32 accumulation. ref: kernels/linear.cuh:5-7,
 // kernels/linear.cu:5-25 (cublasGemmEx, CUBLAS_COMPUTE_32F).
 //
-// These are plain library GEMMs, so they go to hipBLASLt, except with at most 8 rows (a decode
-// step with few sequences), where llmk_linear_rows (gemv.hip) streams the weights itself.
+// With at most 8 rows (a decode step with few sequences) llmk_linear_rows (gemv.hip) streams the
+// weights; 9 to 256 rows of most shapes run this library's tiles (gemm_tiles.hip); the rest,
+// prompts above all, are plain library GEMMs and go to hipBLASLt.
 // Viewed column-major, the row-major buffers are W: [in x out] (ld in), x: [in x T] (ld in),
 // y: [out x T] (ld out), and y = op_T(W) * x -- the same formulation as the reference's cuBLAS
 // call.
@@ -32,6 +33,7 @@
 #include <tuple>
 #include <vector>
 
+#include "gemm_tiles.hpp"
 #include "llmk.h"
 
 namespace {
@@ -219,6 +221,12 @@ extern "C" int llmk_linear(llmk_blas* h, const uint16_t* x, const uint16_t* w, u
   if (!x || !w || !y) return LLMK_ERR_INVALID_VALUE;
   if (rows_kernel_applies(x, w, T, in_features))
     return llmk_linear_rows(x, w, y, T, in_features, out_features, stream);
+  if (llmk::tiles_apply(x, w, y, T, in_features, out_features)) {
+    const llmk::TilePlan plan = llmk::tiles_plan(T, in_features, out_features,
+                                                 kWorkspaceBytes / sizeof(float), true);
+    return llmk::tiles_linear(plan, x, w, y, static_cast<float*>(h->workspace), T, in_features,
+                              out_features, static_cast<hipStream_t>(stream));
+  }
   Plan p;
   {
     std::lock_guard<std::mutex> lock(h->mu);
@@ -244,7 +252,9 @@ extern "C" int llmk_blas_tune(llmk_blas* h, const uint16_t* x, const uint16_t* w
                               int T, int in_features, int out_features, void* stream) {
   if (!h || T <= 0 || in_features <= 0 || out_features <= 0 || !x || !w || !y)
     return LLMK_ERR_INVALID_VALUE;
-  if (rows_kernel_applies(x, w, T, in_features)) return LLMK_OK;  // no library plan to choose
+  if (rows_kernel_applies(x, w, T, in_features) ||
+      llmk::tiles_apply(x, w, y, T, in_features, out_features))
+    return LLMK_OK;  // no library plan to choose
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(static_cast<hipStream_t>(stream), &cap) != hipSuccess ||
       cap != hipStreamCaptureStatusNone)

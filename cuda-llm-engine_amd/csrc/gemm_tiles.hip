@@ -1,0 +1,347 @@
+// y[T, out] = x[T, in] W^T for 9 to 256 rows on the matrix cores: W stored [out, in] row-major (a
+// PyTorch Linear without bias), fp16 in and out, fp32 accumulation. ref: kernels/linear.cu:5-25
+// (cublasGemmEx with CUBLAS_COMPUTE_32F).
+//
+// What bounds it: with this few rows a projection is a stream over W (a few MB to a few hundred)
+// between two fixed costs, about 2.3 us from a block's start to its first stage in LDS and 1 to 3
+// from its last store to the next kernel's first instruction. hipBLASLt's plans spend 11 us and
+// more on the small matrices. So every shape is cut into about one block per CU:
+//   - a block computes BN features x BM rows. Stages of BK of the in dimension go from memory
+//     straight to LDS (global_load_lds_dwordx4, no registers), ST of them in a ring with one
+//     barrier per stage: wait for the stage's loads (counted, the later ones stay in flight),
+//     barrier, issue the loads of the slot that the barrier has freed, read, multiply;
+//   - 16-byte pieces of a row are XOR-ed by the row's low bits, on the way in by the lane's choice
+//     of source and on the way out in the address, so that a fragment read is free of bank
+//     conflicts;
+//   - the KW sets of a block's waves take different slices of each stage and meet in LDS after the
+//     last one, so a wave's accumulators cover a large tile (fewer LDS reads per product) however
+//     small the block's tile is;
+//   - blocks start at different stages of the in dimension. Rows are a power of two apart, so
+//     blocks in step would all read from the same few memory channels: 16384 x 2048 at 40 rows
+//     16.3 -> 14.5 us;
+//   - a long in dimension over few features is also cut over blocks (splits): fp32 partial sums,
+//     added in split order by the consumer or by k_tiles_reduce;
+//   - the row tiles of one feature tile run on one XCD, next to each other: W crosses HBM once.
+// The product is W x^T (v_mfma_f32_16x16x32_f16, A: 16 features, B: 16 rows of x), so a lane ends
+// up with 4 consecutive features of one row. Same box, cold W, inside a graph, us, hipBLASLt's
+// first choice (tuned) -> here:
+//   in x out        40 rows              64 rows             128 rows            256 rows
+//   2048 x 3072     11.8 (8.7) -> 7.4    12.0 (8.9) -> 7.9   14.6 (10.7) -> 10.0  13.4 (13.5) -> 12.0
+//   2048 x 2048     11.3 (7.2) -> 7.0    11.7 (7.4) -> 7.4   11.2 (8.4) -> 7.5    12.0 (10.4) -> 9.6
+//   2048 x 16384    18.6 (18.2) -> 14.5  18.9 (18.4) -> 15.3 21.7 (21.8) -> 20.9  30.1 (30.3) -> 26.4
+//   8192 x 2048     14.5 (14.3) -> 12.8  22.8 (16.4) -> 13.8 21.7 (20.9) -> 16.1  27.9 (27.4) -> 21.5
+#include "gemm_tiles.hpp"
+
+#include "common.hpp"
+
+namespace llmk {
+namespace {
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) void lds_void;
+
+__device__ __forceinline__ void dma16(const void* g, void* wave_base) {
+  __builtin_amdgcn_global_load_lds(g, (lds_void*)wave_base, 16, 0, 0);
+}
+// s_waitcnt vmcnt(VM), the other counters left alone (gfx9 fields).
+template <int VM>
+__device__ __forceinline__ void wait_vm() {
+  static_assert(VM >= 0 && VM < 64, "waitcnt field range");
+  __builtin_amdgcn_s_waitcnt((VM & 15) | ((VM >> 4) << 14) | (7 << 4) | (15 << 8));
+}
+// s_barrier alone: __syncthreads() would wait for every load in flight.
+__device__ __forceinline__ void raw_barrier() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// What a launch does with the product.
+enum Epi : int {
+  kStore = 0,    // y[t][j] = r16(sum)
+  kPartial = 1,  // partial[split][t][j] = sum
+};
+
+struct TileArgs {
+  const f16* x;  // [T, in]
+  const f16* w;  // [out, in]
+  f16* y;        // [T, out]
+  float* partial;  // [splits, T, out]
+  int T, in, out, splits;
+  int row_tiles, col_tiles;
+};
+
+// TM x TN 16 x 16 products per wave, WGM x WGN waves over the block's rows and features, KW sets
+// of them over each stage; KI 32-wide products per wave and stage, ST stages.
+template <int TM_, int TN_, int WGM_, int WGN_, int KW_, int KI_, int ST_, int WAVES_PER_SIMD_>
+struct Tile {
+  static constexpr int TM = TM_, TN = TN_, WGM = WGM_, WGN = WGN_, KW = KW_, KI = KI_, ST = ST_;
+  static constexpr int WAVES_PER_SIMD = WAVES_PER_SIMD_;
+  static constexpr int BM = 16 * TM * WGM, BN = 16 * TN * WGN, BK = 32 * KW * KI;
+  static constexpr int NW = WGM * WGN * KW;          // waves
+  static constexpr int PIECES = BK / 8;              // 16-byte pieces of a row in a stage
+  static constexpr int ROWS_PER_LOAD = 64 / PIECES;  // rows that one wave's load covers
+  static constexpr int LOADS = (BM + BN) / ROWS_PER_LOAD / NW;  // per wave and stage
+  static constexpr int STAGE = (BM + BN) * BK;                  // halves
+  static constexpr size_t RING = (size_t)ST * STAGE * sizeof(f16);
+  static constexpr size_t MEET = KW == 1 ? 0 : (size_t)NW * TM * TN * 64 * sizeof(f32x4);
+  static constexpr size_t LDS = RING > MEET ? RING : MEET;
+  static_assert(PIECES >= 8, "the XOR moves a piece within 8");
+  static_assert(LOADS * NW * ROWS_PER_LOAD == BM + BN && BN % ROWS_PER_LOAD == 0, "whole loads");
+  static_assert((ST - 1) * LOADS < 64, "the wait counts every load in flight");
+  static_assert(LDS <= 160 * 1024, "LDS of a CU");
+};
+
+template <class C, int EPI>
+__global__ void __launch_bounds__(64 * C::NW, C::WAVES_PER_SIMD) k_tiles(TileArgs a) {
+  constexpr int TM = C::TM, TN = C::TN, KW = C::KW, BK = C::BK, ST = C::ST, LOADS = C::LOADS;
+  extern __shared__ __align__(16) f16 lds[];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int kw = wave % KW, wn = wave / KW % C::WGN, wm = wave / KW / C::WGN;
+
+  // Block b runs on XCD b % 8: consecutive tiles go to one XCD, a feature tile's row tiles first.
+  const int per_split = a.row_tiles * a.col_tiles, total = per_split * a.splits;
+  const int xcd = blockIdx.x % 8, q = total / 8, r = total % 8;
+  const int id = xcd * q + (xcd < r ? xcd : r) + (int)blockIdx.x / 8;
+  const int split = id / per_split, tile = id % per_split;
+  const int tn = tile / a.row_tiles, tm = tile % a.row_tiles;
+  const int stages = a.in / BK;
+  const int s0 = (int)((long long)stages * split / a.splits);
+  const int n = (int)((long long)stages * (split + 1) / a.splits) - s0;
+  const int first = n > 0 ? tn % n : 0;  // the stage that this feature tile starts with
+
+  // The wave's loads of a stage: LDS rows (BN features, then BM rows of x) in groups of
+  // ROWS_PER_LOAD. Features and rows past the end repeat the last one and are not stored.
+  const f16* src[LOADS];
+#pragma unroll
+  for (int i = 0; i < LOADS; ++i) {
+    const int group = wave * LOADS + i;
+    const int row = group * C::ROWS_PER_LOAD + lane / C::PIECES;
+    const f16* base;
+    if (group * C::ROWS_PER_LOAD < C::BN) {
+      const int j = tn * C::BN + row;
+      base = a.w + (size_t)(j < a.out ? j : a.out - 1) * a.in;
+    } else {
+      const int t = tm * C::BM + row - C::BN;
+      base = a.x + (size_t)(t < a.T ? t : a.T - 1) * a.in;
+    }
+    src[i] = base + (size_t)s0 * BK + ((lane % C::PIECES) ^ (row & 7)) * 8;
+  }
+  auto issue = [&](int s) {
+    f16* to = lds + (s % ST) * C::STAGE + wave * LOADS * 512;
+    const int at = s + first < n ? s + first : s + first - n;
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) dma16(src[i] + (size_t)at * BK, to + i * 512);
+  };
+
+  f32x4 acc[TN][TM];
+#pragma unroll
+  for (int i = 0; i < TN; ++i)
+#pragma unroll
+    for (int j = 0; j < TM; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int s = 0; s < ST - 1; ++s)
+    if (s < n) issue(s);
+  const int l16 = lane & 15, lq = lane >> 4;
+  for (int s = 0; s < n; ++s) {
+    // Issued so far: min(n, s + ST - 1) stages; stage s has landed when those after it are all
+    // that is left.
+    if (s + ST - 1 <= n)
+      wait_vm<(ST - 2) * LOADS>();
+    else
+      wait_vm<0>();
+    raw_barrier();
+    if (s + ST - 1 < n) issue(s + ST - 1);  // the slot of stage s - 1, read by every wave
+    const f16* st = lds + (s % ST) * C::STAGE;
+#pragma unroll
+    for (int ki = 0; ki < C::KI; ++ki) {
+      const int piece = (kw * C::KI + ki) * 4 + lq;
+      f16x8 wf[TN], xf[TM];
+#pragma unroll
+      for (int i = 0; i < TN; ++i) {
+        const int row = (wn * TN + i) * 16 + l16;
+        wf[i] = as_h8(ld16(st + row * BK + (piece ^ (row & 7)) * 8));
+      }
+#pragma unroll
+      for (int j = 0; j < TM; ++j) {
+        const int row = C::BN + (wm * TM + j) * 16 + l16;
+        xf[j] = as_h8(ld16(st + row * BK + (piece ^ (row & 7)) * 8));
+      }
+#pragma unroll
+      for (int i = 0; i < TN; ++i)
+#pragma unroll
+        for (int j = 0; j < TM; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wf[i], xf[j], acc[i][j], 0, 0, 0);
+    }
+  }
+
+  // The KW sets meet in LDS: set kw adds up the vectors v with v % KW == kw.
+  f32x4* meet = reinterpret_cast<f32x4*>(lds) + (size_t)(wave - kw) * TN * TM * 64 + lane;
+  if constexpr (KW > 1) {
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int j = 0; j < TM; ++j) meet[((size_t)kw * TN * TM + i * TM + j) * 64] = acc[i][j];
+    __syncthreads();
+  }
+  auto total_of = [&](int i, int j) {
+    if constexpr (KW == 1) return acc[i][j];
+    const int v = i * TM + j;
+    f32x4 sum = meet[(size_t)v * 64];
+#pragma unroll
+    for (int k = 1; k < KW; ++k) sum = sum + meet[((size_t)k * TN * TM + v) * 64];
+    return sum;
+  };
+#pragma unroll
+  for (int i = 0; i < TN; ++i)
+#pragma unroll
+    for (int j = 0; j < TM; ++j) {
+      if ((i * TM + j) % KW != kw) continue;
+      const int t = tm * C::BM + (wm * TM + j) * 16 + l16;
+      const int f = tn * C::BN + (wn * TN + i) * 16 + lq * 4;
+      if (t >= a.T || f >= a.out) continue;
+      const f32x4 sum = total_of(i, j);
+      if constexpr (EPI == kPartial) {
+        *reinterpret_cast<f32x4*>(a.partial + ((size_t)split * a.T + t) * a.out + f) = sum;
+      } else {
+        const f16x2 lo = {(f16)sum[0], (f16)sum[1]}, hi = {(f16)sum[2], (f16)sum[3]};
+        uint2 v;
+        v.x = __builtin_bit_cast(uint32_t, lo);
+        v.y = __builtin_bit_cast(uint32_t, hi);
+        *reinterpret_cast<uint2*>(a.y + (size_t)t * a.out + f) = v;
+      }
+    }
+}
+
+// y = r16 of the partial sums, added in split order: 4 values per thread (out is a multiple of 4).
+__global__ void __launch_bounds__(256)
+k_tiles_reduce(const float* __restrict__ partial, f16* __restrict__ y, size_t n, int splits) {
+  const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
+  if (i >= n) return;
+  f32x4 sum = *reinterpret_cast<const f32x4*>(partial + i);
+  for (int s = 1; s < splits; ++s)
+    sum = sum + *reinterpret_cast<const f32x4*>(partial + (size_t)s * n + i);
+  const f16x2 lo = {(f16)sum[0], (f16)sum[1]}, hi = {(f16)sum[2], (f16)sum[3]};
+  uint2 v;
+  v.x = __builtin_bit_cast(uint32_t, lo);
+  v.y = __builtin_bit_cast(uint32_t, hi);
+  *reinterpret_cast<uint2*>(y + i) = v;
+}
+
+// The tile shapes, smallest first, features x rows.
+using T32x32 = Tile<2, 2, 1, 1, 4, 1, 4, 2>;
+using T32x64 = Tile<4, 2, 1, 1, 4, 1, 3, 2>;
+using T64x64 = Tile<2, 2, 2, 2, 2, 2, 3, 2>;
+using T64x128 = Tile<4, 2, 2, 2, 2, 1, 3, 4>;
+using T128x128 = Tile<4, 2, 2, 4, 1, 2, 4, 2>;
+constexpr int kTiles = 5;
+// What a launch takes by shape, in us: start + per_stage * (128-wide stages per CU - free), with
+// the blocks in rounds of one per CU. Fitted to sweeps of every shape and split count over 9 to 256
+// rows of 2048 x 3072, 2048, 16384 and 128256, 8192 x 2048, 4096 x 24576, 12288 x 4096, 1024 x
+// 8192 and 4096 x 1024; the choice it leads to is within 5% of the fastest in all but a few.
+struct Shape {
+  int bm, bn;
+  float start, per_stage;
+  int free;  // stages that the launch's start hides
+};
+constexpr Shape kShapes[kTiles] = {{32, 32, 4.5f, 0.25f, 3},
+                                   {64, 32, 4.5f, 0.42f, 0},
+                                   {64, 64, 4.4f, 0.64f, 0},
+                                   {128, 64, 5.0f, 0.82f, 0},
+                                   {128, 128, 4.5f, 1.25f, 0}};
+
+long long tile_blocks(const Shape& s, int T, int out) {
+  return (long long)((T + s.bm - 1) / s.bm) * ((out + (long long)s.bn - 1) / s.bn);
+}
+
+template <class C, int EPI>
+int tile_launch(TileArgs a, hipStream_t stream) {
+  a.row_tiles = (a.T + C::BM - 1) / C::BM;
+  a.col_tiles = (a.out + C::BN - 1) / C::BN;
+  // More than 64 KiB of LDS has to be asked for, once per kernel and device.
+  static int granted[64];
+  int dev = 0;
+  int st = (int)hipGetDevice(&dev);
+  if (st != LLMK_OK) return st;
+  if (dev < 0 || dev >= 64) return LLMK_ERR_UNSUPPORTED;
+  if (!__atomic_load_n(&granted[dev], __ATOMIC_RELAXED)) {
+    st = (int)hipFuncSetAttribute(reinterpret_cast<const void*>(k_tiles<C, EPI>),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)C::LDS);
+    if (st != LLMK_OK) return st;
+    __atomic_store_n(&granted[dev], 1, __ATOMIC_RELAXED);
+  }
+  const long long blocks = (long long)a.row_tiles * a.col_tiles * a.splits;
+  if (blocks > 0x7FFFFFFFLL) return LLMK_ERR_UNSUPPORTED;
+  return launch(k_tiles<C, EPI>, dim3((unsigned)blocks), dim3(64 * C::NW), C::LDS, stream, a);
+}
+
+template <int EPI>
+int tiles_launch(int tile, const TileArgs& a, hipStream_t stream) {
+  switch (tile) {
+    case 0: return tile_launch<T32x32, EPI>(a, stream);
+    case 1: return tile_launch<T32x64, EPI>(a, stream);
+    case 2: return tile_launch<T64x64, EPI>(a, stream);
+    case 3: return tile_launch<T64x128, EPI>(a, stream);
+    default: return tile_launch<T128x128, EPI>(a, stream);
+  }
+}
+
+}  // namespace
+
+// Past 128 rows, products of more than one round of the largest tile stay with hipBLASLt, whose
+// larger tiles win there: 128256 outputs at 256 rows 181 us against 206 here, 4096 x 24576 at 160
+// rows 59 against 74 (at 128 rows 131 against 130 and 54 against 47).
+bool tiles_apply(const void* x, const void* w, const void* y, int T, int in, int out) {
+  if (T <= LLMK_LINEAR_ROWS_MAX || T > kTilesMaxRows || in % 128 != 0 || out % 4 != 0 ||
+      !aligned16(x) || !aligned16(w) || (reinterpret_cast<uintptr_t>(y) & 7u) != 0)
+    return false;
+  return T <= 128 || tile_blocks(kShapes[kTiles - 1], T, out) <= device_cus();
+}
+
+// The cheapest shape and split count by the model at kShapes. Splits add their partial sums, written
+// and read at 6 TB/s, and with reduce_launch a launch of 2.5 us.
+TilePlan tiles_plan(int T, int in, int out, size_t max_floats, bool reduce_launch) {
+  const int cus = device_cus() > 0 ? device_cus() : 256;
+  TilePlan best = {0, 1};
+  float best_us = 0.0f;
+  for (int tile = 0; tile < kTiles; ++tile) {
+    const Shape& s = kShapes[tile];
+    const long long blocks = tile_blocks(s, T, out);
+    for (int splits = 1; splits <= 8 && splits <= in / 128; splits *= 2) {
+      const double floats = (double)splits * T * out;
+      if (splits > 1 && floats > (double)max_floats) break;
+      const long long rounds = (blocks * splits + cus - 1) / cus;
+      const float stages = (float)rounds * (float)in / 128.0f / (float)splits - (float)s.free;
+      float us = s.start + s.per_stage * (stages > 0.0f ? stages : 0.0f);
+      if (splits > 1) us += (float)(floats * 8.0 / 6e6) + (reduce_launch ? 2.5f : 0.0f);
+      if ((tile == 0 && splits == 1) || us < best_us) {
+        best = {tile, splits};
+        best_us = us;
+      }
+    }
+  }
+  return best;
+}
+
+int tiles_linear(const TilePlan& p, const uint16_t* x, const uint16_t* w, uint16_t* y,
+                 float* partial, int T, int in, int out, hipStream_t stream) {
+  TileArgs a = {};
+  a.x = reinterpret_cast<const f16*>(x);
+  a.w = reinterpret_cast<const f16*>(w);
+  a.y = reinterpret_cast<f16*>(y);
+  a.partial = partial;
+  a.T = T;
+  a.in = in;
+  a.out = out;
+  a.splits = p.splits;
+  if (p.splits == 1) return tiles_launch<kStore>(p.tile, a, stream);
+  const int st = tiles_launch<kPartial>(p.tile, a, stream);
+  if (st != LLMK_OK) return st;
+  const size_t n = (size_t)T * out;
+  return launch(k_tiles_reduce, dim3(ceil_div(n, 1024)), dim3(256), 0, stream,
+                (const float*)partial, a.y, n, p.splits);
+}
+
+}  // namespace llmk

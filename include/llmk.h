@@ -301,9 +301,11 @@ LLMK_API void llmk_blas_destroy(llmk_blas* h);
 
 /* y[T, out_features] = x[T, in_features] * W^T, W stored [out_features, in_features] row-major
  * (a PyTorch Linear without bias); fp16 in and out, fp32 accumulation. With T <= 8,
- * in_features % 512 == 0 and x, W 16-byte aligned it runs llmk_linear_rows; otherwise the first
- * call of a shape takes hipBLASLt's heuristic choice (make that call outside graph capture) and
- * later calls only enqueue. ref: kernels/linear.cuh:5-7, kernels/linear.cu:5-25 (linear;
+ * in_features % 512 == 0 and x, W 16-byte aligned it runs llmk_linear_rows. With 9 to 256 rows,
+ * in_features % 128 == 0, out_features % 4 == 0, x, W 16-byte and y 8-byte aligned it runs this
+ * library's tiles (partial sums in the handle's workspace), except, past 128 rows, products so
+ * wide that hipBLASLt is faster. Otherwise the first call of a shape takes hipBLASLt's heuristic
+ * choice (make that call outside graph capture) and later calls only enqueue. ref: kernels/linear.cuh:5-7, kernels/linear.cu:5-25 (linear;
  * cublasHandle_t -> llmk_blas*). */
 LLMK_API int llmk_linear(llmk_blas* h, const uint16_t* x, const uint16_t* w, uint16_t* y, int T,
                          int in_features, int out_features, void* stream);
@@ -353,7 +355,8 @@ LLMK_API int llmk_linear_rows_qkv_rope_scatter(const uint16_t* x, const uint16_t
 
 /* Chooses the algorithm of one shape by timing hipBLASLt's heuristic candidates with cold
  * caches, on `stream` with these operands (y is overwritten; synchronous; not while the stream
- * is capturing). Later llmk_linear calls of the shape use it. New entry point. */
+ * is capturing). Later llmk_linear calls of the shape use it. Nothing to do, and nothing done, for
+ * calls that llmk_linear runs with this library's kernels. New entry point. */
 LLMK_API int llmk_blas_tune(llmk_blas* h, const uint16_t* x, const uint16_t* w, uint16_t* y,
                             int T, int in_features, int out_features, void* stream);
 

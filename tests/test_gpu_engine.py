@@ -68,6 +68,40 @@ def test_linear_matches_oracle(llmk, orc, blas, T, K, N):
     assert bad == 0 and exact > 0.9
 
 
+# Rows and shapes at the edges of the tiles: one row or feature past a tile, fewer stages of the in
+# dimension than the ring holds, a stage count that no split divides, more than one XCD round, and
+# shapes that the tiles refuse (in not a multiple of 128, out not of 4, one round of the largest
+# tile passed).
+TILE_CASES = [(9, 128, 4), (9, 256, 3072), (31, 1152, 36), (32, 128, 2056), (33, 8192, 68),
+              (64, 640, 4100), (65, 2048, 8196), (127, 384, 128), (128, 8192, 132),
+              (129, 4096, 1028), (200, 2048, 16380), (255, 1152, 260), (256, 8192, 2052),
+              (256, 256, 16384), (257, 256, 64), (12, 192, 64), (40, 256, 66), (130, 128, 32772)]
+
+
+@pytest.mark.parametrize("T,K,N", TILE_CASES)
+def test_linear_tiles_match_oracle(llmk, orc, blas, T, K, N):
+    """9 to 256 rows, against the oracle by the reference's projection rule (ref:
+    tests/test_linear.cu:47), with a value past the output watched; a row of infinities stays in
+    its own row of the output."""
+    rng = np.random.default_rng(0x5EED0300 + 7 * T + N)
+    x, w = normal_f16(rng, (T, K)), normal_f16(rng, (N, K), std=0.05)
+    y = torch.full((T * N + 8,), float("nan"), dtype=torch.float16, device=DEV)
+    print(f"linear T={T} K={K} N={N}", flush=True)
+    llmk.linear(blas, dev(x), dev(w), y, T, K, N)
+    torch.cuda.synchronize()
+    got = host(y)
+    assert np.all(got[T * N:] == 0x7E00), "write past the output"
+    bad, exact = linear_rule(got[:T * N], orc.linear(x, w, T, K, N, threads=16).ravel())
+    assert bad == 0 and exact > 0.9, (bad, exact)
+    x[T // 2] = 0x7C00
+    llmk.linear(blas, dev(x), dev(w), y, T, K, N)
+    torch.cuda.synchronize()
+    again = host(y)[:T * N].reshape(T, N)
+    others = np.arange(T) != T // 2
+    assert np.array_equal(again[others], got[:T * N].reshape(T, N)[others])
+    assert not np.isfinite(again[T // 2].view(np.float16)).any()
+
+
 @pytest.mark.parametrize("K,N", [(2048, 3072), (2048, 2048), (8192, 2048), (512, 1000),
                                  (2048, 16384), (2048, 20480), (2048, 16392), (1536, 16384),
                                  (1024, 13)])
