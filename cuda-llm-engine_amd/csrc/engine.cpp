@@ -15,13 +15,16 @@
 // row-major matrices):
 //   qkv    = normed @ wqkv^T                      (one GEMM for the three projections)
 //   q, K, V: llmk_qkv_rope_scatter                (RoPE on q and k, K/V into the pools)
-//   attn   = llmk_attention_decode_fast(q, pools)
+//   attn   = attention of q over the pools        (decode rows and prompt tiles)
 //   proj   = attn @ wo^T
 //   residual += proj; normed = rmsnorm(residual)  (llmk_add_rmsnorm)
 //   gu     = normed @ wgu^T                       (one GEMM for gate and up)
 //   act    = swiglu(gu)                           (llmk_swiglu_rows)
 //   proj   = act @ wdown^T
 //   residual += proj; normed = rmsnorm(residual) with the next layer's (or the final) norm
+// With 9 to 256 rows the GEMMs are gemm_tiles.hip's and the element-wise steps between them run in
+// their epilogues: RoPE + scatter and SwiGLU on the product's registers, the residual add and the
+// norm over the product's split pieces. With at most 8 rows the same goes for gemv.hip's.
 // Then the logits of the selected rows, lm head = the embedding matrix (tied weights, ref:
 // engine/batched.cu:117), and their argmax.
 //
@@ -43,6 +46,7 @@
 #include <vector>
 
 #include "attention.hpp"
+#include "gemm_tiles.hpp"
 #include "llmk.h"
 
 namespace {
@@ -93,6 +97,9 @@ struct llmk_engine {
            *proj = nullptr, *gu = nullptr, *act = nullptr, *fin = nullptr, *logits = nullptr;
   int32_t* next = nullptr;
   float* ws = nullptr;
+  // The pass's rotation pairs (cos, sin in fp16) and pool rows, made once for its layers.
+  uint32_t* cos_sin = nullptr;
+  long long* pool_rows = nullptr;
 
   // Pages the longest attention of the rows last set reads (position / 16 + 1).
   int rows_span = 0;
@@ -217,6 +224,11 @@ int find_tiles(int n, const int32_t* positions, const int32_t* tables, int max_p
   return count;
 }
 
+// The attention's workspace, which also holds a split projection's partial sums.
+size_t workspace_floats(const llmk_engine* e) {
+  return llmk_attention_decode_fast_workspace_floats(e->max_rows, e->cfg.n_heads, kMaxSplits);
+}
+
 void carve_activations(llmk_engine* e, Carver& c) {
   const llmk_model_config& m = e->cfg;
   const size_t R = e->max_rows, H = m.hidden;
@@ -232,8 +244,9 @@ void carve_activations(llmk_engine* e, Carver& c) {
   e->fin = c.take<uint16_t>(R * H);
   e->logits = c.take<uint16_t>(R * m.vocab);
   e->next = c.take<int32_t>(R);
-  e->ws = c.take<float>(llmk_attention_decode_fast_workspace_floats(e->max_rows, m.n_heads,
-                                                                    kMaxSplits));
+  e->ws = c.take<float>(workspace_floats(e));
+  e->cos_sin = c.take<uint32_t>(R * 32);
+  e->pool_rows = c.take<long long>(R);
 }
 
 void release(llmk_engine* e) {
@@ -671,6 +684,27 @@ extern "C" int llmk_engine_set_option(llmk_engine* e, int option, int value) {
   }
 }
 
+// A projection back to the residual stream and the norm after it: residual += fp16(in W^T),
+// normed = rmsnorm(residual) with norm_w. On this library's tiles the norm adds up the product's
+// split pieces itself.
+static int project_add_norm(llmk_engine* e, const uint16_t* in, const uint16_t* w,
+                            const uint16_t* norm_w, int n, int in_features, void* stream) {
+  const int H = e->cfg.hidden;
+  const size_t floats = workspace_floats(e);
+  if (H <= llmk::kPartialNormMaxHidden && (size_t)n * H <= floats &&
+      llmk::tiles_apply(nullptr, nullptr, nullptr, n, in_features, H)) {
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const llmk::TilePlan plan = llmk::tiles_plan(n, in_features, H, floats, false);
+    const int st = llmk::tiles_partial(plan, in, w, e->ws, n, in_features, H, s);
+    if (st != LLMK_OK) return st;
+    return llmk::add_rmsnorm_partial(e->ws, plan.splits, e->x, norm_w, e->normed, n, H,
+                                     e->cfg.eps, s);
+  }
+  const int st = llmk_linear(e->blas, in, w, e->proj, n, in_features, H, stream);
+  if (st != LLMK_OK) return st;
+  return llmk_add_rmsnorm(e->x, e->proj, norm_w, e->normed, n, H, e->cfg.eps, stream);
+}
+
 // The pass of llmk_engine_forward, its arguments checked and num_splits resolved.
 static int forward_pass(llmk_engine* e, int n, int n_logit_rows, int num_splits, bool tiled,
                         void* s) {
@@ -686,26 +720,49 @@ static int forward_pass(llmk_engine* e, int n, int n_logit_rows, int num_splits,
   } while (0)
   LLMK_TRY(llmk_embedding_lookup(e->embed, e->tokens, e->x, n, H, s));
   if (L > 0) LLMK_TRY(llmk_rmsnorm(e->x, e->layers[0].attn_norm, e->normed, n, H, m.eps, s));
+  const bool qkv_tiles = llmk::tiles_apply(nullptr, nullptr, nullptr, n, H, e->qkvdim);
+  const bool gu_tiles = llmk::tiles_apply(nullptr, nullptr, nullptr, n, H, 2 * m.inter);
+  if (qkv_tiles && L > 0)
+    LLMK_TRY(llmk::rope_rows(e->positions, e->tables, e->inv_freq, e->max_pages, n, e->cos_sin,
+                             e->pool_rows, static_cast<hipStream_t>(s)));
   for (int l = 0; l < L; ++l) {
     const LayerPtrs& w = e->layers[l];
-    LLMK_TRY(llmk_linear(e->blas, e->normed, w.wqkv, e->qkv, n, H, e->qkvdim, s));
-    LLMK_TRY(llmk_qkv_rope_scatter(e->qkv, e->qkvdim, e->q, e->k_pool[l], e->v_pool[l],
-                                   e->tables, e->positions, e->inv_freq, n, e->max_pages, kPage,
-                                   m.n_heads, m.n_kv_heads, m.head_dim, s));
+    if (qkv_tiles) {
+      llmk::RopeTarget to;
+      to.q_out = reinterpret_cast<_Float16*>(e->q);
+      to.k_pool = reinterpret_cast<_Float16*>(e->k_pool[l]);
+      to.v_pool = reinterpret_cast<_Float16*>(e->v_pool[l]);
+      to.cos_sin = e->cos_sin;
+      to.pool_rows = e->pool_rows;
+      to.n_heads = m.n_heads;
+      to.n_kv_heads = m.n_kv_heads;
+      LLMK_TRY(llmk::tiles_qkv_rope_scatter(e->normed, w.wqkv, to, n, H,
+                                            static_cast<hipStream_t>(s)));
+    } else {
+      LLMK_TRY(llmk_linear(e->blas, e->normed, w.wqkv, e->qkv, n, H, e->qkvdim, s));
+      LLMK_TRY(llmk_qkv_rope_scatter(e->qkv, e->qkvdim, e->q, e->k_pool[l], e->v_pool[l],
+                                     e->tables, e->positions, e->inv_freq, n, e->max_pages, kPage,
+                                     m.n_heads, m.n_kv_heads, m.head_dim, s));
+    }
     LLMK_TRY(attention(e, l, n, tiled, num_splits, s));
-    LLMK_TRY(llmk_linear(e->blas, e->attn, w.wo, e->proj, n, e->qdim, H, s));
-    LLMK_TRY(llmk_add_rmsnorm(e->x, e->proj, w.mlp_norm, e->normed, n, H, m.eps, s));
-    LLMK_TRY(llmk_linear(e->blas, e->normed, w.wgu, e->gu, n, H, 2 * m.inter, s));
-    LLMK_TRY(llmk_swiglu_rows(e->gu, e->act, n, m.inter, s));
-    LLMK_TRY(llmk_linear(e->blas, e->act, w.wdown, e->proj, n, m.inter, H, s));
-    if (l + 1 < L)
-      LLMK_TRY(llmk_add_rmsnorm(e->x, e->proj, e->layers[l + 1].attn_norm, e->normed, n, H,
-                                m.eps, s));
+    LLMK_TRY(project_add_norm(e, e->attn, w.wo, w.mlp_norm, n, e->qdim, s));
+    if (gu_tiles) {
+      LLMK_TRY(llmk::tiles_swiglu(e->normed, w.wgu, e->act, n, H, m.inter,
+                                  static_cast<hipStream_t>(s)));
+    } else {
+      LLMK_TRY(llmk_linear(e->blas, e->normed, w.wgu, e->gu, n, H, 2 * m.inter, s));
+      LLMK_TRY(llmk_swiglu_rows(e->gu, e->act, n, m.inter, s));
+    }
+    if (l + 1 < L || all_rows)
+      LLMK_TRY(project_add_norm(e, e->act, w.wdown,
+                                l + 1 < L ? e->layers[l + 1].attn_norm : e->final_norm, n,
+                                m.inter, s));
+    else
+      LLMK_TRY(llmk_linear(e->blas, e->act, w.wdown, e->proj, n, m.inter, H, s));
   }
   const uint16_t* lm_in = e->normed;
   if (all_rows) {
-    if (L > 0) LLMK_TRY(llmk_add_rmsnorm(e->x, e->proj, e->final_norm, e->normed, n, H, m.eps, s));
-    else LLMK_TRY(llmk_rmsnorm(e->x, e->final_norm, e->normed, n, H, m.eps, s));
+    if (L == 0) LLMK_TRY(llmk_rmsnorm(e->x, e->final_norm, e->normed, n, H, m.eps, s));
   } else if (nl > 0) {
     // Only the selected rows go through the final norm and the lm head: gather them (the
     // embedding gather with the residual as the table), then normalise.

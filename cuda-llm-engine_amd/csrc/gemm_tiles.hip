@@ -32,12 +32,13 @@
 //   8192 x 2048     14.5 (14.3) -> 12.8  22.8 (16.4) -> 13.8 21.7 (20.9) -> 16.1  27.9 (27.4) -> 21.5
 #include "gemm_tiles.hpp"
 
-#include "common.hpp"
+#include "layer_ops.hpp"
 
 namespace llmk {
 namespace {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void lds_void;
 
 __device__ __forceinline__ void dma16(const void* g, void* wave_base) {
@@ -56,11 +57,19 @@ __device__ __forceinline__ void raw_barrier() {
   asm volatile("" ::: "memory");
 }
 
-// What a launch does with the product.
+__device__ __forceinline__ void store4(f16* to, f16x4 v) {
+  *reinterpret_cast<uint2*>(to) = __builtin_bit_cast(uint2, v);
+}
+
+// What a launch does with the product. The last two take pairs of features, whose sums the tile's
+// feature order brings into one lane, and every row of W in one block (no splits).
 enum Epi : int {
   kStore = 0,    // y[t][j] = r16(sum)
   kPartial = 1,  // partial[split][t][j] = sum
+  kSwiglu = 2,   // features j (gate) and out / 2 + j (up) -> y[t][j] = r16(r16(silu(g)) * u)
+  kRope = 3,     // q, k, v heads of 64: RoPE on q and k, k and v into the paged pools
 };
+constexpr bool paired(int epi) { return epi == kSwiglu || epi == kRope; }
 
 struct TileArgs {
   const f16* x;  // [T, in]
@@ -69,7 +78,22 @@ struct TileArgs {
   float* partial;  // [splits, T, out]
   int T, in, out, splits;
   int row_tiles, col_tiles;
+  RopeTarget rope;  // kRope
 };
+
+// The feature at LDS row `row` of the tile's BN features; tile number `tile`. Paired: 16
+// features of a wave's 32 are the first halves of its pairs, the next 16 the second halves.
+template <class C, int EPI>
+__device__ __forceinline__ int feature_of(int tile, int row, int out) {
+  if constexpr (paired(EPI)) {
+    static_assert(C::TN == 2, "a pair's halves are the wave's two feature tiles");
+    const int group = tile * C::WGN + row / 32, half = row / 16 % 2, c = row % 16;
+    return EPI == kSwiglu ? half * (out / 2) + 16 * group + c
+                          : 64 * (group / 2) + 32 * half + 16 * (group % 2) + c;
+  } else {
+    return tile * C::BN + row;
+  }
+}
 
 // TM x TN 16 x 16 products per wave, WGM x WGN waves over the block's rows and features, KW sets
 // of them over each stage; KI 32-wide products per wave and stage, ST stages.
@@ -120,7 +144,7 @@ __global__ void __launch_bounds__(64 * C::NW, C::WAVES_PER_SIMD) k_tiles(TileArg
     const int row = group * C::ROWS_PER_LOAD + lane / C::PIECES;
     const f16* base;
     if (group * C::ROWS_PER_LOAD < C::BN) {
-      const int j = tn * C::BN + row;
+      const int j = feature_of<C, EPI>(tn, row, a.out);
       base = a.w + (size_t)(j < a.out ? j : a.out - 1) * a.in;
     } else {
       const int t = tm * C::BM + row - C::BN;
@@ -194,25 +218,99 @@ __global__ void __launch_bounds__(64 * C::NW, C::WAVES_PER_SIMD) k_tiles(TileArg
     for (int k = 1; k < KW; ++k) sum = sum + meet[((size_t)k * TN * TM + v) * 64];
     return sum;
   };
+  if constexpr (paired(EPI)) {
+    const int group = tn * C::WGN + wn;
+    // The set's pairs of vectors: j = kw, kw + KW, ...
+    constexpr int NJ = (TM + KW - 1) / KW;
+    f16x4 lo[NJ], hi[NJ];
 #pragma unroll
-  for (int i = 0; i < TN; ++i)
+    for (int m = 0; m < NJ; ++m) {
+      const int j = kw + KW * m;
+      f32x4 a0 = f32x4{0.0f, 0.0f, 0.0f, 0.0f}, a1 = a0;
+      if constexpr (KW == 1) {
+        a0 = acc[0][m];
+        a1 = acc[1][m];
+      } else if (j < TM) {
+        a0 = total_of(0, j);
+        a1 = total_of(1, j);
+      }
 #pragma unroll
-    for (int j = 0; j < TM; ++j) {
-      if ((i * TM + j) % KW != kw) continue;
-      const int t = tm * C::BM + (wm * TM + j) * 16 + l16;
-      const int f = tn * C::BN + (wn * TN + i) * 16 + lq * 4;
-      if (t >= a.T || f >= a.out) continue;
-      const f32x4 sum = total_of(i, j);
-      if constexpr (EPI == kPartial) {
-        *reinterpret_cast<f32x4*>(a.partial + ((size_t)split * a.T + t) * a.out + f) = sum;
-      } else {
-        const f16x2 lo = {(f16)sum[0], (f16)sum[1]}, hi = {(f16)sum[2], (f16)sum[3]};
-        uint2 v;
-        v.x = __builtin_bit_cast(uint32_t, lo);
-        v.y = __builtin_bit_cast(uint32_t, hi);
-        *reinterpret_cast<uint2*>(a.y + (size_t)t * a.out + f) = v;
+      for (int e = 0; e < 4; ++e) {
+        lo[m][e] = (f16)a0[e];
+        hi[m][e] = (f16)a1[e];
       }
     }
+    if constexpr (EPI == kSwiglu) {
+      constexpr int NV = (NJ + 1) / 2;  // vectors of 8 gates; a spare half holds 1.0
+      u32x4 g[NV], sv[NV];
+#pragma unroll
+      for (int v = 0; v < NV; ++v) {
+        f16x8 gh;
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          gh[e] = 2 * v + e / 4 < NJ ? lo[2 * v + e / 4 < NJ ? 2 * v + e / 4 : 0][e % 4] : (f16)1.0f;
+        g[v] = as_u4(gh);
+      }
+      silu_vectors<NV>(g, sv);
+#pragma unroll
+      for (int m = 0; m < NJ; ++m) {
+        const int j = kw + KW * m, t = tm * C::BM + (wm * TM + j) * 16 + l16;
+        const int col = 16 * group + 4 * lq;
+        if (j >= TM || t >= a.T || col >= a.out / 2) continue;
+        const f16x8 sh = as_h8(sv[m / 2]);
+        f16x4 o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = sh[4 * (m % 2) + e] * hi[m][e];
+        store4(a.y + (size_t)t * (a.out / 2) + col, o);
+      }
+    } else {
+      const RopeTarget& to = a.rope;
+      const int h = group / 2, i0 = 16 * (group % 2) + 4 * lq;
+      const int nq = to.n_heads, nkv = to.n_kv_heads;
+      if (h >= nq + 2 * nkv) return;
+#pragma unroll
+      for (int m = 0; m < NJ; ++m) {
+        const int j = kw + KW * m, t = tm * C::BM + (wm * TM + j) * 16 + l16;
+        if (j >= TM || t >= a.T) continue;
+        f16x4 x1 = lo[m], x2 = hi[m];
+        if (h < nq + nkv) {
+          const u32x4 cs = ld16(to.cos_sin + (size_t)t * 32 + i0);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const f16x2 p = __builtin_bit_cast(f16x2, elem(cs, e));
+            x1[e] = lo[m][e] * p[0] - hi[m][e] * p[1];
+            x2[e] = hi[m][e] * p[0] + lo[m][e] * p[1];
+          }
+        }
+        f16* dst;
+        if (h < nq) {
+          dst = to.q_out + ((size_t)t * nq + h) * 64;
+        } else {
+          const int hk = h < nq + nkv ? h - nq : h - nq - nkv;
+          dst = (h < nq + nkv ? to.k_pool : to.v_pool) +
+                ((size_t)to.pool_rows[t] * nkv + hk) * 64;
+        }
+        store4(dst + i0, x1);
+        store4(dst + i0 + 32, x2);
+      }
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int j = 0; j < TM; ++j) {
+        if ((i * TM + j) % KW != kw) continue;
+        const int t = tm * C::BM + (wm * TM + j) * 16 + l16;
+        const int f = tn * C::BN + (wn * TN + i) * 16 + lq * 4;
+        if (t >= a.T || f >= a.out) continue;
+        const f32x4 sum = total_of(i, j);
+        if constexpr (EPI == kPartial)
+          *reinterpret_cast<f32x4*>(a.partial + ((size_t)split * a.T + t) * a.out + f) = sum;
+        else
+          store4(a.y + (size_t)t * a.out + f,
+                 f16x4{(f16)sum[0], (f16)sum[1], (f16)sum[2], (f16)sum[3]});
+      }
+  }
 }
 
 // y = r16 of the partial sums, added in split order: 4 values per thread (out is a multiple of 4).
@@ -223,11 +321,7 @@ k_tiles_reduce(const float* __restrict__ partial, f16* __restrict__ y, size_t n,
   f32x4 sum = *reinterpret_cast<const f32x4*>(partial + i);
   for (int s = 1; s < splits; ++s)
     sum = sum + *reinterpret_cast<const f32x4*>(partial + (size_t)s * n + i);
-  const f16x2 lo = {(f16)sum[0], (f16)sum[1]}, hi = {(f16)sum[2], (f16)sum[3]};
-  uint2 v;
-  v.x = __builtin_bit_cast(uint32_t, lo);
-  v.y = __builtin_bit_cast(uint32_t, hi);
-  *reinterpret_cast<uint2*>(y + i) = v;
+  store4(y + i, f16x4{(f16)sum[0], (f16)sum[1], (f16)sum[2], (f16)sum[3]});
 }
 
 // The tile shapes, smallest first, features x rows.
@@ -325,23 +419,78 @@ TilePlan tiles_plan(int T, int in, int out, size_t max_floats, bool reduce_launc
   return best;
 }
 
-int tiles_linear(const TilePlan& p, const uint16_t* x, const uint16_t* w, uint16_t* y,
-                 float* partial, int T, int in, int out, hipStream_t stream) {
+namespace {
+
+TileArgs tile_args(const uint16_t* x, const uint16_t* w, int T, int in, int out, int splits) {
   TileArgs a = {};
   a.x = reinterpret_cast<const f16*>(x);
   a.w = reinterpret_cast<const f16*>(w);
-  a.y = reinterpret_cast<f16*>(y);
-  a.partial = partial;
   a.T = T;
   a.in = in;
   a.out = out;
-  a.splits = p.splits;
+  a.splits = splits;
+  return a;
+}
+
+}  // namespace
+
+int tiles_linear(const TilePlan& p, const uint16_t* x, const uint16_t* w, uint16_t* y,
+                 float* partial, int T, int in, int out, hipStream_t stream) {
+  TileArgs a = tile_args(x, w, T, in, out, p.splits);
+  a.y = reinterpret_cast<f16*>(y);
+  a.partial = partial;
   if (p.splits == 1) return tiles_launch<kStore>(p.tile, a, stream);
   const int st = tiles_launch<kPartial>(p.tile, a, stream);
   if (st != LLMK_OK) return st;
   const size_t n = (size_t)T * out;
   return launch(k_tiles_reduce, dim3(ceil_div(n, 1024)), dim3(256), 0, stream,
                 (const float*)partial, a.y, n, p.splits);
+}
+
+int tiles_partial(const TilePlan& p, const uint16_t* x, const uint16_t* w, float* partial, int T,
+                  int in, int out, hipStream_t stream) {
+  TileArgs a = tile_args(x, w, T, in, out, p.splits);
+  a.partial = partial;
+  return tiles_launch<kPartial>(p.tile, a, stream);
+}
+
+int tiles_swiglu(const uint16_t* x, const uint16_t* w_gate_up, uint16_t* act, int T, int in,
+                 int inter, hipStream_t stream) {
+  TileArgs a = tile_args(x, w_gate_up, T, in, 2 * inter, 1);
+  a.y = reinterpret_cast<f16*>(act);
+  return tiles_launch<kSwiglu>(tiles_plan(T, in, 2 * inter, 0, false).tile, a, stream);
+}
+
+int tiles_qkv_rope_scatter(const uint16_t* x, const uint16_t* w_qkv, const RopeTarget& to, int T,
+                           int in, hipStream_t stream) {
+  const int out = (to.n_heads + 2 * to.n_kv_heads) * 64;
+  TileArgs a = tile_args(x, w_qkv, T, in, out, 1);
+  a.rope = to;
+  return tiles_launch<kRope>(tiles_plan(T, in, out, 0, false).tile, a, stream);
+}
+
+// Two rows per block, a thread per rotation pair: a pass's (cos, sin) pairs and pool rows, once
+// for all layers.
+namespace {
+__global__ void __launch_bounds__(64)
+k_rope_rows(const int* __restrict__ positions, const int* __restrict__ tables,
+            const float* __restrict__ inv_freq, int max_pages, int n, f16x2* cos_sin,
+            long long* pool_rows) {
+  const int t = blockIdx.x * 2 + (threadIdx.x >> 5), i = threadIdx.x & 31;
+  if (t >= n) return;
+  const int pos = positions[t];
+  f16 c, s;
+  cos_sin_f16((float)pos * inv_freq[i], &c, &s);
+  cos_sin[(size_t)t * 32 + i] = f16x2{c, s};
+  if (i == 0)
+    pool_rows[t] = (long long)tables[(size_t)t * max_pages + pos / 16] * 16 + pos % 16;
+}
+}  // namespace
+
+int rope_rows(const int32_t* positions, const int32_t* tables, const float* inv_freq,
+              int max_pages, int n, void* cos_sin, long long* pool_rows, hipStream_t stream) {
+  return launch(k_rope_rows, dim3(ceil_div((size_t)n, 2)), dim3(64), 0, stream, positions, tables,
+                inv_freq, max_pages, n, static_cast<f16x2*>(cos_sin), pool_rows);
 }
 
 }  // namespace llmk

@@ -13,6 +13,7 @@
 // of the normal cache-allocation path measured 9% faster at [8192, 2048] than plain accesses. Rows wider than
 // 64 * 8 * 16 = 8192 values take a block-per-row kernel that reads the row twice (the second
 // time from L2).
+#include "gemm_tiles.hpp"
 #include "layer_ops.hpp"
 
 namespace llmk {
@@ -199,6 +200,96 @@ static int rmsnorm_launch(const f16* x, f16* resid, const f16* w, f16* out, int 
 #undef LLMK_NORM_CASE
   return launch(k_rmsnorm_block<FUSED>, dim3(n_rows), dim3(256), 0, stream, x, resid, w, out,
                 vpr, hf, eps);
+}
+
+// residual add + RMSNorm over the S pieces of a split projection (gemm_tiles.hip): x of a row is
+// their sum in split order, rounded to fp16. One block per row and 8 values per thread and step
+// (VPT steps): the S pieces are 32 bytes each and few rows have to keep every CU busy, so a row's
+// loads are spread over 4 waves and issued together. It takes the place of a reduction launch
+// (2.5 us) and of an fp16 copy of the product.
+template <int VPT, int S>
+__global__ void __launch_bounds__(256)
+k_add_rmsnorm_partial(const float* __restrict__ partial, size_t piece, f16* resid,
+                      const f16* __restrict__ w, f16* __restrict__ out, int vpr, float hidden_f,
+                      float eps) {
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+  __shared__ float part[4];
+  const size_t base = (size_t)blockIdx.x * vpr * 8;
+  f32x4 p[VPT][S][2];
+  f16x8 h[VPT], wv[VPT];
+#pragma unroll
+  for (int k = 0; k < VPT; ++k) {
+    const int v = threadIdx.x + 256 * k;
+    if (v >= vpr) continue;
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+        p[k][s][q] = *reinterpret_cast<const f32x4*>(partial + s * piece + base + 8 * v + 4 * q);
+    h[k] = as_h8(ld16(resid + base + 8 * v));
+    wv[k] = as_h8(ld16(w + 8 * v));
+  }
+  float ss = 0.0f;
+#pragma unroll
+  for (int k = 0; k < VPT; ++k) {
+    const int v = threadIdx.x + 256 * k;
+    if (v >= vpr) continue;
+    f16x8 x;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      f32x4 sum = p[k][0][q];
+#pragma unroll
+      for (int s = 1; s < S; ++s) sum = sum + p[k][s][q];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) x[4 * q + e] = (f16)sum[e];
+    }
+    h[k] = h[k] + x;
+    st16(resid + base + 8 * v, as_u4(h[k]));
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float f = (float)h[k][j];
+      ss = ss + f * f;
+    }
+  }
+  ss = wave_sum(ss);
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = ss;
+  lds_barrier();
+  const float total = (part[0] + part[1]) + (part[2] + part[3]);
+  const float inv = 1.0f / __builtin_sqrtf(total / hidden_f + eps);
+#pragma unroll
+  for (int k = 0; k < VPT; ++k) {
+    const int v = threadIdx.x + 256 * k;
+    if (v >= vpr) continue;
+    f16x8 a;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) a[j] = (f16)((float)h[k][j] * inv);
+    st16(out + base + 8 * v, as_u4(wv[k] * a));
+  }
+}
+
+int add_rmsnorm_partial(const float* partial, int splits, uint16_t* residual, const uint16_t* w,
+                        uint16_t* out, int rows, int hidden, float eps, hipStream_t stream) {
+  if (hidden % 8 != 0 || hidden > kPartialNormMaxHidden) return LLMK_ERR_SHAPE;
+  const int vpr = hidden / 8, vpt = (vpr + 255) / 256;
+  auto go = [&](auto kern) {
+    return launch(kern, dim3((unsigned)rows), dim3(256), 0, stream, partial,
+                  (size_t)rows * hidden, reinterpret_cast<f16*>(residual),
+                  reinterpret_cast<const f16*>(w), reinterpret_cast<f16*>(out), vpr,
+                  (float)hidden, eps);
+  };
+#define LLMK_PARTIAL_NORM(S)                                          \
+  case S:                                                             \
+    return vpt <= 1   ? go(k_add_rmsnorm_partial<1, S>)               \
+           : vpt <= 2 ? go(k_add_rmsnorm_partial<2, S>)               \
+                      : go(k_add_rmsnorm_partial<4, S>)
+  switch (splits) {
+    LLMK_PARTIAL_NORM(1);
+    LLMK_PARTIAL_NORM(2);
+    LLMK_PARTIAL_NORM(4);
+    LLMK_PARTIAL_NORM(8);
+    default: return LLMK_ERR_UNSUPPORTED;
+  }
+#undef LLMK_PARTIAL_NORM
 }
 
 }  // namespace llmk
