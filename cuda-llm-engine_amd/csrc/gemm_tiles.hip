@@ -324,11 +324,15 @@ k_tiles_reduce(const float* __restrict__ partial, f16* __restrict__ y, size_t n,
   store4(y + i, f16x4{(f16)sum[0], (f16)sum[1], (f16)sum[2], (f16)sum[3]});
 }
 
-// The tile shapes, smallest first, features x rows.
+// The tile shapes, smallest first, features x rows. More waves to a tile issue its loads faster (a
+// wave alone gets about 12 bytes a ns into LDS, 16 waves 110 together): 32x64 with 8 waves of 32x32
+// instead of 4 of 64x32 10.2 -> 9.6 us (2048 x 3072, 128 rows), 64x128 with 16 waves in one block
+// instead of 8 in each of two 20.3 -> 19.2 (2048 x 16384, 128 rows). 128x128 takes 26 us at 256
+// rows of that matrix with 4, 8 or 16 waves, one block or two, and any ring depth.
 using T32x32 = Tile<2, 2, 1, 1, 4, 1, 4, 2>;
-using T32x64 = Tile<4, 2, 1, 1, 4, 1, 3, 2>;
+using T32x64 = Tile<2, 2, 2, 1, 4, 1, 4, 4>;
 using T64x64 = Tile<2, 2, 2, 2, 2, 2, 3, 2>;
-using T64x128 = Tile<4, 2, 2, 2, 2, 1, 3, 4>;
+using T64x128 = Tile<2, 2, 4, 2, 2, 2, 3, 4>;
 using T128x128 = Tile<4, 2, 2, 4, 1, 2, 4, 2>;
 constexpr int kTiles = 5;
 // What a launch takes by shape, in us: start + per_stage * (128-wide stages per CU - free), with
@@ -341,9 +345,9 @@ struct Shape {
   int free;  // stages that the launch's start hides
 };
 constexpr Shape kShapes[kTiles] = {{32, 32, 4.5f, 0.25f, 3},
-                                   {64, 32, 4.5f, 0.42f, 0},
+                                   {64, 32, 4.5f, 0.43f, 5},
                                    {64, 64, 4.4f, 0.64f, 0},
-                                   {128, 64, 5.0f, 0.82f, 0},
+                                   {128, 64, 5.0f, 0.80f, 0},
                                    {128, 128, 4.5f, 1.25f, 0}};
 
 long long tile_blocks(const Shape& s, int T, int out) {
