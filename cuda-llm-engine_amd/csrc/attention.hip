@@ -762,7 +762,8 @@ k_attn_merge(const float* __restrict__ part_o, const float2* __restrict__ part_m
   store_out(out, seq, h, n_heads, A, L);
 }
 
-// Merge for many pieces per sequence (the small-batch grid's short runs). Grid (n_heads, n_seq)
+// Merge for many pieces per sequence (the small-batch grid's short runs, and the page-balanced
+// grid's segments of a few sequences). Grid (n_heads, n_seq)
 // of one-wave blocks: block (h, seq) merges the pieces of query head h of sequence seq, for
 // every sequence that has more than one. (One wave per block rather than four per 256-thread
 // block puts the few waves of a small batch on more CUs: same box, bits unchanged, 1 x 2048
@@ -949,6 +950,14 @@ int short_run_launch(const AttnArgs& a, int groups, int pps, hipStream_t s) {
 // blocks lose (8.84 us at 1 sequence).
 constexpr int kTwoWavePairs = 8;
 
+// Expected segments per sequence from which the page-balanced grid's pieces go to
+// k_attn_merge_many, which folds 32 in one round trip where k_attn_merge takes 4 at a time in
+// turn. Same box, 8 kv heads, both kernels, us, k_attn_merge -> k_attn_merge_many: 1 x 16384 (64
+// segments, capped at 31) 20.7 -> 16.6, 5 x U[1, 16384] (13) 27.9 -> 25.8, 16 x U[1, 8192] (8)
+// 32.1 -> 30.0, 24 x U[1, 2048] (5) 17.5 -> 17.3; 32 x U[1, 2048] (4) 18.4 -> 18.5, 64 x U[1, 2048]
+// (2) 30.0 -> 31.6, 256 x U[1, 2048] (1) 97.4 -> 105.6.
+constexpr int kManyPieces = 5;
+
 // Whether a call in kv groups of the given number takes the short-run grid: its splits are at most
 // kShortRunPages pages long and its (sequence, kv group) pairs at most kSplitGridPairs.
 bool short_runs(const AttnArgs& a, int groups) {
@@ -974,6 +983,11 @@ int attn_launch(const AttnArgs& a, hipStream_t s) {
                     0, s, a.lens, a.tables, a.n_seq, a.max_pages, a.n_heads, a.n_kv_heads,
                     a.num_splits, blocks, a.q, a.k_pool, a.v_pool, a.out, a.part_o, a.part_ml);
     if (st != 0) return st;
+    // A sequence has about blocks / n_seq segments, num_splits - 1 at most.
+    if (blocks >= (long long)kManyPieces * a.n_seq && a.num_splits > kManyPieces)
+      return launch(k_attn_merge_many, dim3((unsigned)a.n_heads, (unsigned)a.n_seq), dim3(64), 0,
+                    s, a.part_o, a.part_ml, a.lens, a.out, a.max_pages, a.n_heads, a.num_splits,
+                    0);
     const dim3 mgrid((unsigned)((a.n_heads + 7) / 8), (unsigned)a.n_seq);
     return launch(k_attn_merge, mgrid, dim3(64), 0, s, a.part_o, a.part_ml, a.lens, a.out,
                   a.max_pages, a.n_heads, a.num_splits, 0);
