@@ -22,7 +22,7 @@
 //   act    = swiglu(gu)                           (llmk_swiglu_rows)
 //   proj   = act @ wdown^T
 //   residual += proj; normed = rmsnorm(residual) with the next layer's (or the final) norm
-// With 9 to 256 rows the GEMMs are gemm_tiles.hip's and the element-wise steps between them run in
+// With 9 to 512 rows most GEMMs are gemm_tiles.hip's and the element-wise steps between them run in
 // their epilogues: RoPE + scatter and SwiGLU on the product's registers, the residual add and the
 // norm over the product's split pieces. With at most 8 rows the same goes for gemv.hip's.
 // Then the logits of the selected rows, lm head = the embedding matrix (tied weights, ref:
@@ -692,7 +692,7 @@ static int project_add_norm(llmk_engine* e, const uint16_t* in, const uint16_t* 
   const int H = e->cfg.hidden;
   const size_t floats = workspace_floats(e);
   if (H <= llmk::kPartialNormMaxHidden && (size_t)n * H <= floats &&
-      llmk::tiles_apply(nullptr, nullptr, nullptr, n, in_features, H)) {
+      llmk::tiles_apply(nullptr, nullptr, nullptr, n, in_features, H, true)) {
     hipStream_t s = static_cast<hipStream_t>(stream);
     const llmk::TilePlan plan = llmk::tiles_plan(n, in_features, H, floats, false);
     const int st = llmk::tiles_partial(plan, in, w, e->ws, n, in_features, H, s);
@@ -720,8 +720,8 @@ static int forward_pass(llmk_engine* e, int n, int n_logit_rows, int num_splits,
   } while (0)
   LLMK_TRY(llmk_embedding_lookup(e->embed, e->tokens, e->x, n, H, s));
   if (L > 0) LLMK_TRY(llmk_rmsnorm(e->x, e->layers[0].attn_norm, e->normed, n, H, m.eps, s));
-  const bool qkv_tiles = llmk::tiles_apply(nullptr, nullptr, nullptr, n, H, e->qkvdim);
-  const bool gu_tiles = llmk::tiles_apply(nullptr, nullptr, nullptr, n, H, 2 * m.inter);
+  const bool qkv_tiles = llmk::tiles_apply(nullptr, nullptr, nullptr, n, H, e->qkvdim, true);
+  const bool gu_tiles = llmk::tiles_apply(nullptr, nullptr, nullptr, n, H, 2 * m.inter, true);
   if (qkv_tiles && L > 0)
     LLMK_TRY(llmk::rope_rows(e->positions, e->tables, e->inv_freq, e->max_pages, n, e->cos_sin,
                              e->pool_rows, static_cast<hipStream_t>(s)));

@@ -3,7 +3,7 @@
 // kernels/linear.cu:5-25 (cublasGemmEx, CUBLAS_COMPUTE_32F).
 //
 // With at most 8 rows (a decode step with few sequences) llmk_linear_rows (gemv.hip) streams the
-// weights; 9 to 256 rows of most shapes run this library's tiles (gemm_tiles.hip); the rest,
+// weights; 9 to 512 rows of most shapes run this library's tiles (gemm_tiles.hip); the rest,
 // prompts above all, are plain library GEMMs and go to hipBLASLt.
 // Viewed column-major, the row-major buffers are W: [in x out] (ld in), x: [in x T] (ld in),
 // y: [out x T] (ld out), and y = op_T(W) * x -- the same formulation as the reference's cuBLAS
@@ -221,7 +221,7 @@ extern "C" int llmk_linear(llmk_blas* h, const uint16_t* x, const uint16_t* w, u
   if (!x || !w || !y) return LLMK_ERR_INVALID_VALUE;
   if (rows_kernel_applies(x, w, T, in_features))
     return llmk_linear_rows(x, w, y, T, in_features, out_features, stream);
-  if (llmk::tiles_apply(x, w, y, T, in_features, out_features)) {
+  if (llmk::tiles_apply(x, w, y, T, in_features, out_features, false)) {
     const llmk::TilePlan plan = llmk::tiles_plan(T, in_features, out_features,
                                                  kWorkspaceBytes / sizeof(float), true);
     return llmk::tiles_linear(plan, x, w, y, static_cast<float*>(h->workspace), T, in_features,
@@ -253,7 +253,7 @@ extern "C" int llmk_blas_tune(llmk_blas* h, const uint16_t* x, const uint16_t* w
   if (!h || T <= 0 || in_features <= 0 || out_features <= 0 || !x || !w || !y)
     return LLMK_ERR_INVALID_VALUE;
   if (rows_kernel_applies(x, w, T, in_features) ||
-      llmk::tiles_apply(x, w, y, T, in_features, out_features))
+      llmk::tiles_apply(x, w, y, T, in_features, out_features, false))
     return LLMK_OK;  // no library plan to choose
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(static_cast<hipStream_t>(stream), &cap) != hipSuccess ||

@@ -1,4 +1,4 @@
-// y[T, out] = x[T, in] W^T for 9 to 256 rows on the matrix cores: W stored [out, in] row-major (a
+// y[T, out] = x[T, in] W^T for 9 to 512 rows on the matrix cores: W stored [out, in] row-major (a
 // PyTorch Linear without bias), fp16 in and out, fp32 accumulation. ref: kernels/linear.cu:5-25
 // (cublasGemmEx with CUBLAS_COMPUTE_32F).
 //
@@ -390,12 +390,17 @@ int tiles_launch(int tile, const TileArgs& a, hipStream_t stream) {
 
 // Past 128 rows, products of more than one round of the largest tile stay with hipBLASLt, whose
 // larger tiles win there: 128256 outputs at 256 rows 181 us against 206 here, 4096 x 24576 at 160
-// rows 59 against 74 (at 128 rows 131 against 130 and 54 against 47).
-bool tiles_apply(const void* x, const void* w, const void* y, int T, int in, int out) {
+// rows 59 against 74 (at 128 rows 131 against 130 and 54 against 47). Past 256 rows so do short
+// products of more than one round of 64 x 64 tiles, unless a launch after them goes too: 2048 x
+// 3072 at 512 rows 15.3 against 16.2, where 2048 x 2048 takes 13.1 against 11.9, 8192 x 2048 37.0
+// against 29.6 and 12288 x 4096 83 against 68.
+bool tiles_apply(const void* x, const void* w, const void* y, int T, int in, int out, bool fused) {
   if (T <= LLMK_LINEAR_ROWS_MAX || T > kTilesMaxRows || in % 128 != 0 || out % 4 != 0 ||
       !aligned16(x) || !aligned16(w) || (reinterpret_cast<uintptr_t>(y) & 7u) != 0)
     return false;
-  return T <= 128 || tile_blocks(kShapes[kTiles - 1], T, out) <= device_cus();
+  const int cus = device_cus();
+  if (T > 128 && tile_blocks(kShapes[kTiles - 1], T, out) > cus) return false;
+  return T <= 256 || fused || in >= 4096 || tile_blocks(kShapes[2], T, out) <= cus;
 }
 
 // The cheapest shape and split count by the model at kShapes. Splits add their partial sums, written

@@ -7,7 +7,7 @@
 
 namespace llmk {
 
-constexpr int kTilesMaxRows = 256;
+constexpr int kTilesMaxRows = 512;
 
 // How a product is cut: the tile shape (an index into gemm_tiles.hip's list) and the number of
 // pieces of the in dimension, whose fp32 partial sums a second pass adds.
@@ -16,8 +16,9 @@ struct TilePlan {
 };
 
 // Whether y[T, out] = x[T, in] W^T runs here: 9 .. kTilesMaxRows rows, in a multiple of 128, out
-// of 4, x and w 16-byte and y 8-byte aligned, and not so wide that hipBLASLt wins.
-bool tiles_apply(const void* x, const void* w, const void* y, int T, int in, int out);
+// of 4, x and w 16-byte and y 8-byte aligned, and not so large that hipBLASLt wins. `fused`: the
+// product's consumer is part of the launch, or adds up its pieces itself.
+bool tiles_apply(const void* x, const void* w, const void* y, int T, int in, int out, bool fused);
 
 // The plan for a shape with at most `max_floats` floats of partial sums. `reduce_launch`: whether
 // the partial sums cost a launch of their own.

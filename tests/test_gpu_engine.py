@@ -75,12 +75,13 @@ def test_linear_matches_oracle(llmk, orc, blas, T, K, N):
 TILE_CASES = [(9, 128, 4), (9, 256, 3072), (31, 1152, 36), (32, 128, 2056), (33, 8192, 68),
               (64, 640, 4100), (65, 2048, 8196), (127, 384, 128), (128, 8192, 132),
               (129, 4096, 1028), (200, 2048, 16380), (255, 1152, 260), (256, 8192, 2052),
-              (256, 256, 16384), (257, 256, 64), (12, 192, 64), (40, 256, 66), (130, 128, 32772)]
+              (256, 256, 16384), (257, 256, 64), (384, 4096, 1028), (512, 8192, 132),
+              (513, 256, 64), (12, 192, 64), (40, 256, 66), (130, 128, 32772)]
 
 
 @pytest.mark.parametrize("T,K,N", TILE_CASES)
 def test_linear_tiles_match_oracle(llmk, orc, blas, T, K, N):
-    """9 to 256 rows, against the oracle by the reference's projection rule (ref:
+    """9 to 512 rows, against the oracle by the reference's projection rule (ref:
     tests/test_linear.cu:47), with a value past the output watched; a row of infinities stays in
     its own row of the output."""
     rng = np.random.default_rng(0x5EED0300 + 7 * T + N)
