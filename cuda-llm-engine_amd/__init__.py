@@ -221,6 +221,27 @@ for _name, (_res, _args) in _SIGS.items():
     _fn.argtypes = _args
 
 
+def _load_fast_calls():
+    """The native calls beside libllmk.so (csrc/fast_calls.c). They answer a status, or None where
+    the checks below have to decide."""
+    import importlib.machinery
+    import importlib.util
+    for suffix in importlib.machinery.EXTENSION_SUFFIXES:
+        path = os.path.join(_HERE, "_fast_calls" + suffix)
+        if os.path.exists(path):
+            spec = importlib.util.spec_from_file_location("_fast_calls", path)
+            mod = importlib.util.module_from_spec(spec)
+            spec.loader.exec_module(mod)
+            mod.setup(torch.Tensor, torch.float16, torch.int32, torch.float32,
+                      torch.cuda.current_device, torch._C._cuda_getCurrentRawStream)
+            return mod
+    raise ImportError(f"_fast_calls not found in {_HERE}: build it first (python -c "
+                      "'import __graft_entry__; __graft_entry__.build()')")
+
+
+_fast = _load_fast_calls()
+
+
 def lib() -> ctypes.CDLL:
     return _lib
 
@@ -300,6 +321,9 @@ def embedding_lookup(table, ids, out, n_tokens: int, hidden: int, stream=None,
 def residual_add(a, b, out, n: int, stream=None) -> None:
     """out = a + b in fp16, out may be a (ref: kernels/residual_add.cuh:6)."""
     fn = "residual_add"
+    st = _fast.residual_add(a, b, out, n, stream)
+    if st is not None:
+        return _check(fn, st)
     pa = _dev(fn, a, torch.float16, n, "a")
     pb = _dev(fn, b, torch.float16, n, "b")
     po = _dev(fn, out, torch.float16, n, "out")
@@ -309,6 +333,9 @@ def residual_add(a, b, out, n: int, stream=None) -> None:
 def rmsnorm(x, w, out, n_rows: int, hidden: int, eps: float, stream=None) -> None:
     """RMSNorm of n_rows rows (ref: kernels/rmsnorm.cuh:6-7)."""
     fn = "rmsnorm"
+    st = _fast.rmsnorm(x, w, out, n_rows, hidden, eps, stream)
+    if st is not None:
+        return _check(fn, st)
     px = _dev(fn, x, torch.float16, n_rows * hidden, "x")
     pw = _dev(fn, w, torch.float16, hidden, "w")
     po = _dev(fn, out, torch.float16, n_rows * hidden, "out")
@@ -318,6 +345,9 @@ def rmsnorm(x, w, out, n_rows: int, hidden: int, eps: float, stream=None) -> Non
 def add_rmsnorm(residual, x, w, out, n_rows: int, hidden: int, eps: float, stream=None) -> None:
     """residual += x (fp16, in place), out = rmsnorm(residual)."""
     fn = "add_rmsnorm"
+    st = _fast.add_rmsnorm(residual, x, w, out, n_rows, hidden, eps, stream)
+    if st is not None:
+        return _check(fn, st)
     pr = _dev(fn, residual, torch.float16, n_rows * hidden, "residual")
     px = _dev(fn, x, torch.float16, n_rows * hidden, "x")
     pw = _dev(fn, w, torch.float16, hidden, "w")
@@ -352,6 +382,9 @@ def rope_apply(q, k, positions, inv_freq, n_tokens: int, n_heads: int, n_kv_head
 def swiglu(gate, up, out, n: int, stream=None) -> None:
     """out = silu(gate) * up (ref: kernels/swiglu.cuh:6)."""
     fn = "swiglu"
+    st = _fast.swiglu(gate, up, out, n, stream)
+    if st is not None:
+        return _check(fn, st)
     pg = _dev(fn, gate, torch.float16, n, "gate")
     pu = _dev(fn, up, torch.float16, n, "up")
     po = _dev(fn, out, torch.float16, n, "out")
@@ -457,6 +490,12 @@ def attention_decode_fast(q, k_pool, v_pool, block_tables, seq_lens, out, worksp
     fits the block table (seq_lens <= max_pages * page_size) and that every page number a
     cached position reads lies inside both pools."""
     fn = "attention_decode_fast"
+    if not _want_checks(check_indices):
+        st = _fast.attention_decode_fast(q, k_pool, v_pool, block_tables, seq_lens, out, workspace,
+                                         n_seq, max_pages, page_size, n_heads, n_kv_heads,
+                                         head_dim, num_splits, stream)
+        if st is not None:
+            return _check(fn, st)
     kvdim = n_kv_heads * head_dim
     pq = _dev(fn, q, torch.float16, n_seq * n_heads * head_dim, "q")
     pk = _dev(fn, k_pool, torch.float16, 0, "k_pool")
@@ -634,6 +673,9 @@ def linear(handle: Blas, x, w, y, T: int, in_features: int, out_features: int,
            stream=None) -> None:
     """y[T, out] = x[T, in] W^T, W [out, in] row-major (ref: kernels/linear.cuh:5-7)."""
     fn = "linear"
+    st = _fast.linear(handle.handle, x, w, y, T, in_features, out_features, stream)
+    if st is not None:
+        return _check(fn, st)
     if T < 0 or in_features <= 0 or out_features <= 0:
         _fail(fn, "T must be >= 0 and the feature counts > 0")
     px = _dev(fn, x, torch.float16, T * in_features, "x")
@@ -679,6 +721,9 @@ def linear_rows_residual(x, w, residual, T: int, in_features: int, out_features:
                          stream=None) -> None:
     """residual += x W^T, rounded as linear then residual_add (``llmk_linear_rows_residual``)."""
     fn = "linear_rows_residual"
+    st = _fast.linear_rows_residual(x, w, residual, T, in_features, out_features, stream)
+    if st is not None:
+        return _check(fn, st)
     px = _dev(fn, x, torch.float16, T * in_features, "x")
     pw = _dev(fn, w, torch.float16, out_features * in_features, "w")
     pr = _dev(fn, residual, torch.float16, T * out_features, "residual")
@@ -690,6 +735,9 @@ def linear_rows_swiglu(x, norm_w, eps: float, w_gate_up, act, T: int, in_feature
                        inter: int, stream=None) -> None:
     """act = swiglu of the gate and up projections of rmsnorm(x) (``llmk_linear_rows_swiglu``)."""
     fn = "linear_rows_swiglu"
+    st = _fast.linear_rows_swiglu(x, norm_w, eps, w_gate_up, act, T, in_features, inter, stream)
+    if st is not None:
+        return _check(fn, st)
     px = _dev(fn, x, torch.float16, T * in_features, "x")
     pw = _dev(fn, w_gate_up, torch.float16, 2 * inter * in_features, "w_gate_up")
     pa = _dev(fn, act, torch.float16, T * inter, "act")
@@ -757,6 +805,9 @@ def qkv_rope_scatter(qkv, ld: int, q_out, k_pool, v_pool, block_tables, position
 def swiglu_rows(gate_up, out, n_rows: int, inter: int, stream=None) -> None:
     """out[r] = swiglu(gate_up[r, :inter], gate_up[r, inter:]) (``llmk_swiglu_rows``)."""
     fn = "swiglu_rows"
+    st = _fast.swiglu_rows(gate_up, out, n_rows, inter, stream)
+    if st is not None:
+        return _check(fn, st)
     if n_rows < 0 or inter <= 0:
         _fail(fn, "n_rows must be >= 0 and inter > 0")
     pg = _dev(fn, gate_up, torch.float16, n_rows * 2 * inter, "gate_up")
