@@ -536,6 +536,34 @@ __device__ __forceinline__ int block_scan(int v, int* red, int* total) {
   return v + before;
 }
 
+// A DPP lane move of an int (lanes without a source get 0).
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp_i32(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xF, false);
+}
+// Inclusive prefix sum over the wave's lanes: row_shr 1, 2, 4, 8 within rows of 16 lanes, then
+// each row's total to the rows after it (row_bcast 15 and 31).
+__device__ __forceinline__ int wave_scan(int v) {
+  v += dpp_i32<0x111, 0xF>(v);
+  v += dpp_i32<0x112, 0xF>(v);
+  v += dpp_i32<0x114, 0xF>(v);
+  v += dpp_i32<0x118, 0xF>(v);
+  v += dpp_i32<0x142, 0xA>(v);
+  v += dpp_i32<0x143, 0xC>(v);
+  return v;
+}
+// Largest of the wave's values, none of them negative.
+__device__ __forceinline__ int wave_max(int v) {
+  auto larger = [](int a, int b) { return a > b ? a : b; };
+  v = larger(v, dpp_i32<0x111, 0xF>(v));
+  v = larger(v, dpp_i32<0x112, 0xF>(v));
+  v = larger(v, dpp_i32<0x114, 0xF>(v));
+  v = larger(v, dpp_i32<0x118, 0xF>(v));
+  v = larger(v, dpp_i32<0x142, 0xA>(v));
+  v = larger(v, dpp_i32<0x143, 0xC>(v));
+  return __builtin_amdgcn_readlane(v, 63);
+}
+
 // Sequences whose page counts a thread keeps in registers during the page-balanced prologue;
 // longer batches read the lengths a second time.
 constexpr int kPrologueTiles = 4;
@@ -598,7 +626,31 @@ k_attn_balanced(const int* __restrict__ seq_lens, const int* __restrict__ block_
       pmax = P > pmax ? P : pmax;
     }
   int U, P_max;
-  block_sum_max(mine, red, &U, &P_max);
+  // With one sequence per thread at most (`single`) the wave's prefix sums are taken here, by lane
+  // moves, and one barrier gives the block's total, maximum and offsets, where the general path
+  // takes 18 dependent LDS shuffles and three more barriers: 5 x U[1, 16384] 29.9 -> 29.4 us, 256 x
+  // U[1, 2048] 89.5 -> 88.9, bits unchanged.
+  const bool single = n_seq <= kThreads;
+  int incl = 0;  // single: units up to and including the thread's sequence
+  if (single) {
+    const int wave = tid >> 6;
+    incl = wave_scan(mine);
+    const int mx = wave_max(pmax);
+    if ((tid & 63) == 63) {
+      red[wave] = incl;
+      red[kWaves + wave] = mx;
+    }
+    lds_barrier();
+    U = P_max = 0;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+      incl += w < wave ? red[w] : 0;
+      U += red[w];
+      P_max = red[kWaves + w] > P_max ? red[kWaves + w] : P_max;
+    }
+  } else {
+    block_sum_max(mine, red, &U, &P_max);
+  }
   const int per = (U + n_blocks - 1) / n_blocks;  // n_blocks == gridDim.x, passed in SGPRs
   const int q_min = P_max > 1 ? (P_max - 1 + num_splits - 3) / (num_splits - 2) : 1;
   const int qp = per > q_min ? per : q_min;
@@ -609,7 +661,12 @@ k_attn_balanced(const int* __restrict__ seq_lens, const int* __restrict__ block_
 
   // The sequence holding unit u0, its first unit and its length.
   int running = 0;
-  const int tiles = (n_seq + kThreads - 1) / kThreads;
+  const int tiles = single ? 0 : (n_seq + kThreads - 1) / kThreads;
+  if (single && mine > 0 && incl - mine <= u0 && u0 < incl) {
+    found[0] = tid;
+    found[1] = incl - mine;
+    found[2] = lv[0];
+  }
   for (int t = 0; t < tiles && running <= u0; ++t) {
     const int s = t * kThreads + tid;
     int S = 0;
@@ -622,10 +679,10 @@ k_attn_balanced(const int* __restrict__ seq_lens, const int* __restrict__ block_
     const int P = seq_pages(S, max_pages);
     const int E = P > 0 ? C + P : 0;
     int tile;
-    const int incl = running + block_scan(E, red, &tile);
-    if (E > 0 && incl - E <= u0 && u0 < incl) {
+    const int upto = running + block_scan(E, red, &tile);
+    if (E > 0 && upto - E <= u0 && u0 < upto) {
       found[0] = s;
-      found[1] = incl - E;
+      found[1] = upto - E;
       found[2] = S;
     }
     running += tile;
