@@ -44,11 +44,13 @@ typedef __attribute__((address_space(3))) void lds_void;
 __device__ __forceinline__ void dma16(const void* g, void* wave_base) {
   __builtin_amdgcn_global_load_lds(g, (lds_void*)wave_base, 16, 0, 0);
 }
-// s_waitcnt vmcnt(VM), the other counters left alone (gfx9 fields).
+// s_waitcnt vmcnt(VM) lgkmcnt(0) (gfx9 fields): at most VM loads still in flight, and every LDS read
+// of the wave returned, so that after the barrier its last stage's slot may be written. The products
+// have used those reads by then, so the second wait costs nothing.
 template <int VM>
 __device__ __forceinline__ void wait_vm() {
   static_assert(VM >= 0 && VM < 64, "waitcnt field range");
-  __builtin_amdgcn_s_waitcnt((VM & 15) | ((VM >> 4) << 14) | (7 << 4) | (15 << 8));
+  __builtin_amdgcn_s_waitcnt((VM & 15) | ((VM >> 4) << 14) | (7 << 4));
 }
 // s_barrier alone: __syncthreads() would wait for every load in flight.
 __device__ __forceinline__ void raw_barrier() {
