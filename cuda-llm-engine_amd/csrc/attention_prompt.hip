@@ -20,7 +20,10 @@
 // 2^12 p that carry 22 bits of it, which doubles that product's 8 instructions to 16 a chunk; the
 // vector work of the softmax (about 6 instructions and one exponential per score) is the larger
 // part. The running maximum is rounded up to a whole number of log2 units: the offset 12 - m is
-// then exact, so the scale 2^12 costs nothing, and rescaling is rarer. The next step's K and V
+// then exact, so the scale 2^12 costs nothing, and rescaling is rarer. That holds for scores below
+// kLargeScore; past it (finite, but far from a trained model's) the same reference is kept as m + f,
+// f the row's largest exponent after m is taken off, and the exponents are made in two steps, so
+// that a row's largest weight stays 2^12 however m rounds. The next step's K and V
 // are in registers while this one is used. At 4000 rows staging alone (LDS writes, V transposed,
 // two barriers) takes 32 of the 156 us, the loads 15.
 #include <math.h>
@@ -39,6 +42,8 @@ constexpr int kVStride = kKeys + 4;  // halves per row of the transposed V: 8-by
                                      // fall on 64 distinct banks, the writes two to a bank
 constexpr float kScoreScale = 0.125f * 1.44269504088896341f;  // 1 / sqrt(64), in log2 units
 constexpr float kWeightLog2 = 12.0f;  // weights are held as 2^12 p
+// Below it 12 - m is exact and a rounded maximum is at most 2^-4 short of the exact one.
+constexpr float kLargeScore = 1048576.0f;
 
 // Splits (prompt_splits): up to one block per CU, of at least two chunks: a few rows far into a
 // sequence would otherwise run on n_kv_heads CUs, chunk after chunk.
@@ -56,7 +61,7 @@ struct Lds {
     };
     struct {  // at the end: all sets of waves but the first
       f32x4 acc[kGroup][8][64];
-      float m[kGroup][64], l[kGroup][64];
+      float m[kGroup][64], f[kGroup][64], l[kGroup][64];
     } merge[PARTS - 1];
   };
   int odd;  // whether some V element is infinite or NaN
@@ -141,7 +146,8 @@ k_attn_prompt(const PromptTile* __restrict__ tiles, const int* __restrict__ posi
   for (int s = 0; s < 4; ++s)
     qf[s] = as_h8(ld16(q + ((size_t)row * n_heads + h) * kHeadDim + 16 * s + 8 * half));
 
-  float m = -INFINITY, l = 0.0f;  // l: this half's positions only
+  // Weights are relative to 2^(m + f), f = 0 while |m| < kLargeScore; l: this half's positions only
+  float m = -INFINITY, f = 0.0f, l = 0.0f;
   f32x16 acc[2];                  // dims 32 d + 8 (i / 4) + 4 half + i % 4
 #pragma unroll
   for (int d = 0; d < 2; ++d)
@@ -211,8 +217,20 @@ k_attn_prompt(const PromptTile* __restrict__ tiles, const int* __restrict__ posi
     float mc = fmaxf(mx[0], mx[1]);
     mc = fmaxf(mc, __shfl_xor(mc, 32));
     const float mn = fmaxf(m, __builtin_ceilf(mc * kScoreScale));
-    if (__builtin_amdgcn_ballot_w64(mn != m)) {
-      const float corr = __builtin_amdgcn_exp2f(m - (mn == -INFINITY ? 0.0f : mn));
+    const float base = mn == -INFINITY ? 0.0f : mn;  // nothing seen yet: every weight is 0
+    float scale = kScoreScale, off = kWeightLog2 - base, fn = 0.0f;
+    if (__builtin_amdgcn_ballot_w64(__builtin_fabsf(base) >= kLargeScore || f != 0.0f)) {
+      const float own = __builtin_fmaf(mc, kScoreScale, -base);
+      if (__builtin_fabsf(base) >= kLargeScore) fn = mn > m ? own : fmaxf(f, own);
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s[t][i] = __builtin_fmaf(s[t][i], kScoreScale, -base) - fn;
+      scale = 1.0f;
+      off = kWeightLog2;
+    }
+    if (__builtin_amdgcn_ballot_w64(mn != m || fn != f)) {
+      const float corr = __builtin_amdgcn_exp2f((m - base) + (f - fn));
       l = l * corr;
 #pragma unroll
       for (int d = 0; d < 2; ++d)
@@ -220,8 +238,7 @@ k_attn_prompt(const PromptTile* __restrict__ tiles, const int* __restrict__ posi
         for (int i = 0; i < 16; ++i) acc[d][i] = acc[d][i] * corr;
     }
     m = mn;
-    // nothing seen yet (mn = -inf): every score is -inf, any finite offset keeps the weights 0
-    const float off = kWeightLog2 - (mn == -INFINITY ? 0.0f : mn);
+    f = fn;
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
@@ -233,7 +250,7 @@ k_attn_prompt(const PromptTile* __restrict__ tiles, const int* __restrict__ posi
 #pragma unroll
           for (int k = 0; k < 2; ++k) {
             p[k] = __builtin_amdgcn_exp2f(
-                __builtin_fmaf(s[t][8 * c + 2 * e + k], kScoreScale, off));
+                __builtin_fmaf(s[t][8 * c + 2 * e + k], scale, off));
             l = l + p[k];
           }
           split_weights(p[0], p[1], hi[e], lo[e]);
@@ -267,14 +284,18 @@ k_attn_prompt(const PromptTile* __restrict__ tiles, const int* __restrict__ posi
         to.acc[w][4 * d + g][lane] = f32x4{acc[d][4 * g], acc[d][4 * g + 1], acc[d][4 * g + 2],
                                            acc[d][4 * g + 3]};
     to.m[w][lane] = m;
+    to.f[w][lane] = f;
     to.l[w][lane] = l;
   }
   __syncthreads();
   if (part > 0 || tok >= count || key0 > pos) return;
-  float M = m;  // finite unless a score is not: the first set saw position key0
+  float M = m, F = f;  // finite unless a score is not: the first set saw position key0
 #pragma unroll
-  for (int p = 0; p < PARTS - 1; ++p) M = fmaxf(M, lds.merge[p].m[w][lane]);
-  const float own = __builtin_amdgcn_exp2f(m - M);
+  for (int p = 0; p < PARTS - 1; ++p) {
+    const float mp = lds.merge[p].m[w][lane], fp = lds.merge[p].f[w][lane];
+    if (mp > M || (mp == M && fp > F)) M = mp, F = fp;
+  }
+  const float own = __builtin_amdgcn_exp2f((m - M) + (f - F));
   l = l * own;
 #pragma unroll
   for (int d = 0; d < 2; ++d)
@@ -283,7 +304,7 @@ k_attn_prompt(const PromptTile* __restrict__ tiles, const int* __restrict__ posi
 #pragma unroll 1
   for (int p = 0; p < PARTS - 1; ++p) {
     const auto& from = lds.merge[p];
-    const float wt = __builtin_amdgcn_exp2f(from.m[w][lane] - M);
+    const float wt = __builtin_amdgcn_exp2f((from.m[w][lane] - M) + (from.f[w][lane] - F));
     l = __builtin_fmaf(from.l[w][lane], wt, l);
 #pragma unroll
     for (int d = 0; d < 2; ++d)
@@ -327,6 +348,14 @@ k_attn_prompt(const PromptTile* __restrict__ tiles, const int* __restrict__ posi
         *reinterpret_cast<uint2*>(dst + 32 * d + 8 * g) = v;
       }
   } else {
+    if (F != 0.0f) {  // pieces meet by M alone
+      const float c = __builtin_amdgcn_exp2f(F);
+      l = l * c;
+#pragma unroll
+      for (int d = 0; d < 2; ++d)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[d][i] = acc[d][i] * c;
+    }
     const size_t idx = ((size_t)row * num_splits + split) * n_heads + h;
     float* dst = part_o + idx * kHeadDim + 4 * half;
 #pragma unroll

@@ -1,0 +1,114 @@
+"""Attention of a prompt's rows in tiles (csrc/attention_prompt.hip) against float64, through a
+one-layer engine whose projections are exact: token vectors of equal magnitudes (the norm turns
+them into signs), projections that are short sums of binary fractions, a RoPE that turns only the
+pair (0, 32), which the queries leave out, an identity output projection and an MLP of zeros. The
+residual is then x + attention, the keys and values are read back from the pools, and the queries
+are known.
+
+A row's result is rounded to fp16 twice (2^-11 each: the attention, then the residual sum) on top
+of fp32 sums; 128 fp32 roundings (2^-17) of sum p |v| are allowed for these."""
+import importlib
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+X = 2.0 ** -14  # magnitude of a token vector's elements
+
+
+class Rows:
+    """n rows of one sequence at positions start .. start + n - 1, each with a token of its own
+    whose signs the caller may set, over cached keys and values that it gives."""
+
+    def __init__(self, n_kv, n, start=0, seed=0):
+        self.rng = np.random.default_rng(seed)
+        self.n_kv, self.n, self.start, self.hidden = n_kv, n, start, 256 * n_kv
+        self.signs = self.rng.choice([-1.0, 1.0], (n, self.hidden))
+        self.signs[:, 0] = 1.0
+        kvd = 64 * n_kv
+        # one row per head: [dims, columns of the token vector]
+        self.wq, self.wk, self.wv = (np.zeros((k, 64, self.hidden)) for k in (4 * n_kv, n_kv, n_kv))
+        self.cached = [np.zeros((start, kvd), np.float16) for _ in range(2)]
+
+    def run(self, llmk, capture=False):
+        """(residual - x, keys, values), in float64."""
+        h, n, n_kv = self.hidden, self.n, self.n_kv
+        end = self.start + n
+        pages = (end + 15) // 16
+        cfg = llmk.ModelConfig(n_layers=1, hidden=h, n_heads=4 * n_kv, n_kv_heads=n_kv, inter=128,
+                               vocab=n, eps=1e-15, rope_theta=1e300)
+        half = lambda a: torch.from_numpy(np.ascontiguousarray(a).astype(np.float16)).cuda()
+        x = self.signs * X
+        e = llmk.Engine(cfg, n, pages, pages)
+        e.set_weights(half(x), half(np.ones(h)), [dict(
+            attn_norm=half(np.ones(h)), wq=half(self.wq.reshape(-1, h)),
+            wk=half(self.wk.reshape(-1, h)), wv=half(self.wv.reshape(-1, h)), wo=half(np.eye(h)),
+            mlp_norm=half(np.ones(h)), w_gate=half(np.zeros((128, h))),
+            w_up=half(np.zeros((128, h))), w_down=half(np.zeros((h, 128))))])
+        table = self.rng.permutation(pages).astype(np.int32)
+        at = table[np.arange(end) // 16] * 16 + np.arange(end) % 16
+        for which, rows in zip((llmk.BUF_K_POOL, llmk.BUF_V_POOL), self.cached):
+            pool = np.full((pages * 16, 64 * n_kv), np.nan, np.float16)
+            pool[at[:self.start]] = rows
+            e.write_pool(which, 0, torch.from_numpy(pool.reshape(-1)))
+        e.set_rows(np.arange(n, dtype=np.int32), np.arange(self.start, end, dtype=np.int32),
+                   np.tile(table, (n, 1)), [n - 1])
+        if capture:  # every row a decode row
+            g, s = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+            torch.cuda.synchronize()
+            with torch.cuda.graph(g, stream=s):
+                e.forward(n, 1, stream=s)
+            g.replay()
+        else:
+            e.forward(n, 1)
+        torch.cuda.synchronize()
+        k, v = (e.pool(w, 0).double().cpu().numpy().reshape(-1, 64 * n_kv)[at]
+                for w in (llmk.BUF_K_POOL, llmk.BUF_V_POOL))
+        return (e.residual(n).double().cpu().numpy().reshape(n, h) - x,
+                k.reshape(end, n_kv, 64), v.reshape(end, n_kv, 64))
+
+    def expected(self, k, v):
+        """(attention, sum p |v|) of every row in float64, [n, 256 n_kv]."""
+        out = np.empty((2, self.n, 4 * self.n_kv, 64))
+        later = np.arange(self.start + self.n)[None, :] > self.start + np.arange(self.n)[:, None]
+        for head in range(4 * self.n_kv):
+            q = self.signs @ self.wq[head].T
+            s = q @ np.nan_to_num(k[:, head // 4]).T / 8
+            s[later] = -np.inf
+            p = np.exp(s - s.max(-1, keepdims=True))
+            p /= p.sum(-1, keepdims=True)
+            vals = v[:, head // 4]
+            out[0, :, head], out[1, :, head] = p @ vals, p @ np.abs(vals)
+        return out.reshape(2, self.n, -1)
+
+    def check(self, llmk, what=""):
+        got, k, v = self.run(llmk)
+        ref, spread = self.expected(k, v)
+        bound = 2.0 ** -10 * np.abs(ref) + 2.0 ** -10 * X + 2.0 ** -17 * spread + 2.0 ** -24
+        worst = np.abs(got - ref) / bound
+        bad = ~(worst <= 1)
+        assert not bad.any(), (what, int(bad.sum()), np.argwhere(bad)[:4], got[bad][:4], ref[bad][:4])
+
+
+# (kv heads, rows, first position), and what they launch: 8 waves over one step; the same in three
+# splits; 16 waves over several steps of one split, the last with wave sets that have no positions.
+LAUNCHES = [(1, 40, 0), (1, 300, 0), (8, 1000, 0)]
+
+
+@pytest.mark.parametrize("n_kv,n,start", LAUNCHES)
+@pytest.mark.parametrize("a,dims,qs,ks", [(128, 8, 4, 0.5), (3584, 8, 4, 2), (12288, 5, 16, 8),
+                                          (12288, 20, 32, 16), (16384, 28, 32, 16),
+                                          (24576, 10, 32, 16)])
+def test_large_finite_scores(llmk, n_kv, n, start, a, dims, qs, ks):
+    """Scores of 2^14.5 to 2^30.3 in units of log2: a weight's exponent is a small difference of
+    large numbers, and a row's largest weight is 1 whichever way these round (by 4, 16 and 47 up
+    and by 63 down in the last four). Every partial sum of q.k is exact, so the scores are too; they
+    differ by multiples of 2 qs ks / 8."""
+    r = Rows(n_kv, n, start, seed=a + n)
+    r.wq[:, 1:1 + dims, 0] = r.wk[:, 1:1 + dims, 0] = a
+    r.wq[:, 40:44, 0] = qs
+    for d in range(4):
+        r.wk[:, 40 + d, 16 + d] = ks
+    r.wv[:, :, 20:36] = r.rng.integers(-4, 5, (n_kv, 64, 16)) / 8
+    r.check(llmk, (a, dims))
