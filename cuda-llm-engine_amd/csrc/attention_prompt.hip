@@ -17,16 +17,23 @@
 //   O^T += V^T P^T (A: V transposed into LDS as it arrives, B: the lane's own 16 weights, whose
 //         position order the A reads follow).
 // Weights stay 32-bit values: each enters the second product as hi + lo, two fp16 halves of
-// 2^12 p that carry 22 bits of it, which doubles that product's 8 instructions to 16 a chunk; the
-// vector work of the softmax (about 6 instructions and one exponential per score) is the larger
-// part. The running maximum is rounded up to a whole number of log2 units: the offset 12 - m is
-// then exact, so the scale 2^12 costs nothing, and rescaling is rarer. That holds for scores below
+// 2^15 p, which doubles that product's 8 instructions to 16 a chunk; the vector work of the
+// softmax (about 6 instructions and one exponential per score) is the larger part. Down to p =
+// 2^-20 of the row's maximum the halves are as near as the decode kernels' fp32
+// weights, whose exponents are rounded; below, where lo runs out of exponents, what they leave goes through the product once
+// more, 2^39 times as large, which serves to p = 2^-59. Only chunks that hold such a weight pay for
+// it: 1507 rows 33.0 -> 34.1 us for the search, 32.6 -> 59.7 where every chunk does (scores of
+// standard deviation 4). Sums that keep their own registers, or the scores, spill: 50 us.
+// The running maximum is rounded up to a whole number of log2 units: the offset 15 - m is
+// then exact, so the scale 2^15 costs nothing, and rescaling is rarer. That holds for scores below
 // kLargeScore; past it (finite, but far from a trained model's) the same reference is kept as m + f,
 // f the row's largest exponent after m is taken off, and the exponents are made in two steps, so
-// that a row's largest weight stays 2^12 however m rounds. The next step's K and V
-// are in registers while this one is used. At 4000 rows staging alone (LDS writes, V transposed,
-// two barriers) takes 32 of the 156 us, the loads 15.
+// that a row's largest weight stays 2^15 however m rounds. The next step's K and V are in registers
+// while this one is used. At 4000 rows staging alone (LDS writes, V transposed, two barriers) takes
+// 32 of the 156 us, the loads 15.
 #include <math.h>
+
+#include <type_traits>
 
 #include "attention.hpp"
 #include "common.hpp"
@@ -41,9 +48,13 @@ constexpr int kKeys = 64;  // positions per chunk
 constexpr int kVStride = kKeys + 4;  // halves per row of the transposed V: 8-byte reads of 32 rows
                                      // fall on 64 distinct banks, the writes two to a bank
 constexpr float kScoreScale = 0.125f * 1.44269504088896341f;  // 1 / sqrt(64), in log2 units
-constexpr float kWeightLog2 = 12.0f;  // weights are held as 2^12 p
-// Below it 12 - m is exact and a rounded maximum is at most 2^-4 short of the exact one.
+constexpr float kWeightLog2 = 15.0f;  // weights are held as 2^15 p
+// Below it 15 - m is exact and a rounded maximum is at most 2^-4 short of the exact one.
 constexpr float kLargeScore = 1048576.0f;
+// The halves end at 2^-24, so a weight of 2^kLowLog2 (2^-20 of the row's maximum) is off by at most
+// 2^-20 of itself, what rounding its exponent (-16 to -32 there) costs a weight of the decode
+// kernels. Of weights below it at most 2^-25 is left: kRest times that fits.
+constexpr float kLowLog2 = -5.0f, kLowWeight = 0.03125f, kRest = 549755813888.0f;
 
 // Splits (prompt_splits): up to one block per CU, of at least two chunks: a few rows far into a
 // sequence would otherwise run on n_kv_heads CUs, chunk after chunk.
@@ -190,24 +201,35 @@ k_attn_prompt(const PromptTile* __restrict__ tiles, const int* __restrict__ posi
     if (step + STEP < key1) load(step + STEP);
     if (step + kKeys * part >= key1) continue;
 
-    f32x16 s[2];
+    const int own = pos - step - kKeys * part - 4 * half;  // positions past it are masked
+    auto scores = [&](int t) {
+      f32x16 s;
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
+      for (int i = 0; i < 16; ++i) s[i] = 0.0f;
       const int key = kKeys * part + 32 * t + tok;
 #pragma unroll
-      for (int i = 0; i < 16; ++i) s[t][i] = 0.0f;
-#pragma unroll
       for (int c = 0; c < 4; ++c)
-        s[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-            as_h8(lds.k[key][(2 * c + half) ^ (tok & 7)]), qf[c], s[t], 0, 0, 0);
-    }
+        s = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+            as_h8(lds.k[key][(2 * c + half) ^ (tok & 7)]), qf[c], s, 0, 0, 0);
+      return s;
+    };
+    auto mask = [&](f32x16& s, int t) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        if (8 * (i / 4) + i % 4 > own - 32 * t) s[i] = -INFINITY;
+    };
+    f32x16 s[2] = {scores(0), scores(1)};
+    // The lowest score, of positions that the row does not attend to as well.
+    float mi[2] = {s[0][0], s[1][0]};
+#pragma unroll
+    for (int i = 1; i < 16; ++i)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) mi[t] = fminf(mi[t], s[t][i]);
+    float lowest = fminf(mi[0], mi[1]);
+    asm volatile("" : "+v"(lowest));  // now: the scores need not be kept for it
     if (masked) {
-      const int own = pos - step - kKeys * part - 4 * half;  // what follows it is masked
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int i = 0; i < 16; ++i)
-          if (32 * t + 8 * (i / 4) + i % 4 > own) s[t][i] = -INFINITY;
+      for (int t = 0; t < 2; ++t) mask(s[t], t);
     }
     float mx[2] = {s[0][0], s[1][0]};
 #pragma unroll
@@ -215,17 +237,24 @@ k_attn_prompt(const PromptTile* __restrict__ tiles, const int* __restrict__ posi
 #pragma unroll
       for (int t = 0; t < 2; ++t) mx[t] = fmaxf(mx[t], s[t][i]);
     float mc = fmaxf(mx[0], mx[1]);
-    mc = fmaxf(mc, __shfl_xor(mc, 32));
+    const auto halves = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, mc),
+                                                         __builtin_bit_cast(uint32_t, mc), false,
+                                                         false);
+    const uint32_t h0 = halves[0], h1 = halves[1];
+    mc = fmaxf(__builtin_bit_cast(float, h0), __builtin_bit_cast(float, h1));
     const float mn = fmaxf(m, __builtin_ceilf(mc * kScoreScale));
     const float base = mn == -INFINITY ? 0.0f : mn;  // nothing seen yet: every weight is 0
     float scale = kScoreScale, off = kWeightLog2 - base, fn = 0.0f;
-    if (__builtin_amdgcn_ballot_w64(__builtin_fabsf(base) >= kLargeScore || f != 0.0f)) {
-      const float own = __builtin_fmaf(mc, kScoreScale, -base);
-      if (__builtin_fabsf(base) >= kLargeScore) fn = mn > m ? own : fmaxf(f, own);
+    const bool large =
+        __builtin_amdgcn_ballot_w64(__builtin_fabsf(base) >= kLargeScore || f != 0.0f) != 0;
+    if (large) {
+      const float top = __builtin_fmaf(mc, kScoreScale, -base);
+      if (__builtin_fabsf(base) >= kLargeScore) fn = mn > m ? top : fmaxf(f, top);
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int i = 0; i < 16; ++i) s[t][i] = __builtin_fmaf(s[t][i], kScoreScale, -base) - fn;
+      lowest = __builtin_fmaf(lowest, kScoreScale, -base) - fn;
       scale = 1.0f;
       off = kWeightLog2;
     }
@@ -239,35 +268,77 @@ k_attn_prompt(const PromptTile* __restrict__ tiles, const int* __restrict__ posi
     }
     m = mn;
     f = fn;
+    unsigned long long low =
+        __builtin_amdgcn_ballot_w64(__builtin_fmaf(lowest, scale, off) < kLowLog2);
+    asm volatile("" : "+s"(low));
+    // 16 positions into the sums: their weights, or kRest times what the halves of the weights
+    // below kLowWeight leave of them.
+    auto weigh = [&](const f32x16& s, float scale, float off, int t, int c, auto rest) {
+      uint32_t hi[4], lo[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float p[2];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          p[k] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[8 * c + 2 * e + k], scale, off));
+          if constexpr (!rest) l = l + p[k];
+        }
+        split_weights(p[0], p[1], hi[e], lo[e]);
+        if constexpr (rest) {
+          const f16x2 h = __builtin_bit_cast(f16x2, hi[e]), r = __builtin_bit_cast(f16x2, lo[e]);
+#pragma unroll
+          for (int k = 0; k < 2; ++k)
+            p[k] = p[k] < kLowWeight ? ((p[k] - (float)h[k]) - (float)r[k]) * kRest : 0.0f;
+          split_weights(p[0], p[1], hi[e], lo[e]);
+        }
+      }
+      const f16x8 h8 = as_h8(u32x4{hi[0], hi[1], hi[2], hi[3]});
+      const f16x8 l8 = as_h8(u32x4{lo[0], lo[1], lo[2], lo[3]});
+      // element e of the lane's weights is position 16 c + 4 half + e, + 4 from e = 4 on
+#pragma unroll
+      for (int d = 0; d < 2; ++d) {
+        const f16* v = &lds.vt[part][32 * d + tok][32 * t + 16 * c + 4 * half];
+        const uint2 v0 = *reinterpret_cast<const uint2*>(v);
+        const uint2 v1 = *reinterpret_cast<const uint2*>(v + 8);
+        const f16x8 vf = as_h8(u32x4{v0.x, v0.y, v1.x, v1.y});
+        acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, h8, acc[d], 0, 0, 0);
+        acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, l8, acc[d], 0, 0, 0);
+      }
+    };
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int c = 0; c < 2; ++c) {  // 16 positions
-        uint32_t hi[4], lo[4];
+      for (int c = 0; c < 2; ++c) weigh(s[t], scale, off, t, c, std::false_type{});
+    asm volatile("" : "+v"(l));  // now: the weights need not be kept for it
+    if (low) {
+      // The scores are made again, 32 positions at a time, and the sums are scaled instead of the
+      // rest (exactly): the registers of the loop are full.
+      float ref = m;
+      asm volatile("" : "+v"(ref));
+      ref = ref == -INFINITY ? 0.0f : ref;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          float p[2];
+      for (int d = 0; d < 2; ++d)
 #pragma unroll
-          for (int k = 0; k < 2; ++k) {
-            p[k] = __builtin_amdgcn_exp2f(
-                __builtin_fmaf(s[t][8 * c + 2 * e + k], scale, off));
-            l = l + p[k];
-          }
-          split_weights(p[0], p[1], hi[e], lo[e]);
+        for (int i = 0; i < 16; ++i) acc[d][i] = acc[d][i] * kRest;
+#pragma unroll 1
+      for (int t = 0; t < 2; ++t) {
+        f32x16 again = scores(t);
+        if (masked) mask(again, t);
+        if (large) {
+#pragma unroll
+          for (int i = 0; i < 16; ++i)
+            again[i] = __builtin_fmaf(again[i], kScoreScale, -ref) - f;
         }
-        const f16x8 h8 = as_h8(u32x4{hi[0], hi[1], hi[2], hi[3]});
-        const f16x8 l8 = as_h8(u32x4{lo[0], lo[1], lo[2], lo[3]});
-        // element e of the lane's weights is position 16 c + 4 half + e, + 4 from e = 4 on
 #pragma unroll
-        for (int d = 0; d < 2; ++d) {
-          const f16* v = &lds.vt[part][32 * d + tok][32 * t + 16 * c + 4 * half];
-          const uint2 v0 = *reinterpret_cast<const uint2*>(v);
-          const uint2 v1 = *reinterpret_cast<const uint2*>(v + 8);
-          const f16x8 vf = as_h8(u32x4{v0.x, v0.y, v1.x, v1.y});
-          acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, h8, acc[d], 0, 0, 0);
-          acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf, l8, acc[d], 0, 0, 0);
-        }
+        for (int c = 0; c < 2; ++c)
+          weigh(again, large ? 1.0f : kScoreScale, kWeightLog2 - (large ? 0.0f : ref), t, c,
+                std::true_type{});
       }
+#pragma unroll
+      for (int d = 0; d < 2; ++d)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[d][i] = acc[d][i] * (1.0f / kRest);
+    }
   }
   l = l + __shfl_xor(l, 32);
 

@@ -112,3 +112,22 @@ def test_large_finite_scores(llmk, n_kv, n, start, a, dims, qs, ks):
         r.wk[:, 40 + d, 16 + d] = ks
     r.wv[:, :, 20:36] = r.rng.integers(-4, 5, (n_kv, 64, 16)) / 8
     r.check(llmk, (a, dims))
+
+
+@pytest.mark.parametrize("n_kv,n,start", LAUNCHES)
+@pytest.mark.parametrize("key", [7.0, 9.75, 12.5])
+def test_small_weights_keep_their_bits(llmk, n_kv, n, start, key):
+    """Position 0 takes nearly all of every row's weight and its value is zero: the result is made
+    of the others' weights, 2^-20, 2^-28 and 2^-36 of the largest, and their values near 2^14."""
+    r = Rows(n_kv, n, start, seed=n + int(key))
+    r.signs[:, 1] = 1.0
+    r.signs[0, 1] = -1.0
+    r.signs[0, 16:32:2], r.signs[0, 17:32:2] = 1.0, -1.0
+    r.wq[:, 1:5, 0] = 2.0
+    r.wk[:, 1:5, 1] = -key
+    r.wq[:, 10:20, 0] = 0.5
+    r.wk[:, 10:20, 16:26] = np.eye(10) / 2
+    r.wv[:, :, 0] = r.wv[:, :, 1] = 2.0 ** 13
+    pairs = r.rng.integers(0, 2, (n_kv, 64, 4)) * 2.0 ** 10
+    r.wv[:, :, 16:24:2] = r.wv[:, :, 17:24:2] = pairs
+    r.check(llmk, key)
