@@ -3,14 +3,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-namespace llmk {
+#include "prompt_plan.hpp"
 
-// A prompt tile: `count` (1 .. kTileRows) consecutive rows of a pass, at consecutive positions of
-// one sequence, whose block-table rows agree on every page that the last of them reads.
-constexpr int kTileRows = 32;
-struct PromptTile {
-  int32_t row0, count;
-};
+namespace llmk {
 
 struct PromptAttention {
   const uint16_t *q, *k_pool, *v_pool;  // as llmk_attention_decode_fast
@@ -20,16 +15,12 @@ struct PromptAttention {
   uint16_t* out;
   float* workspace;  // llmk_attention_decode_fast's, for num_splits splits (unused with 1)
   int n_rows, n_tiles, max_pages, n_heads, n_kv_heads;
-  int num_splits, pages_per_split;  // split s of a row: pages [s, s + 1) * pages_per_split
+  PromptSplits splits;
 };
 
 // Attention of the rows in `tiles` over all of their cached positions (their own included); rows
 // in no tile are left alone.
 int prompt_attention(const PromptAttention& a, hipStream_t stream);
-
-// Splits for a launch over n_tiles tiles whose longest attention spans `span` pages.
-void prompt_splits(int n_tiles, int n_kv_heads, int span, int max_splits, int* num_splits,
-                   int* pages_per_split);
 
 // Merges the pieces of a sequence-split launch (attention.hip): rows of lens[] cut into
 // ceil(pages / pages_per_split) pieces, those with more than one.

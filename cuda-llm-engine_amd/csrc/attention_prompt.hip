@@ -56,10 +56,6 @@ constexpr float kLargeScore = 1048576.0f;
 // kernels. Of weights below it at most 2^-25 is left: kRest times that fits.
 constexpr float kLowLog2 = -5.0f, kLowWeight = 0.03125f, kRest = 549755813888.0f;
 
-// Splits (prompt_splits): up to one block per CU, of at least two chunks: a few rows far into a
-// sequence would otherwise run on n_kv_heads CUs, chunk after chunk.
-constexpr int kTargetBlocks = 256, kMinSplitPages = 8;
-
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
@@ -449,9 +445,9 @@ constexpr long long kWideBlocks = 512;
 template <int PARTS>
 int tiles_launch(const PromptAttention& a, float2* ml, hipStream_t stream) {
   return launch(k_attn_prompt<PARTS>,
-                dim3((unsigned)a.n_kv_heads, (unsigned)a.num_splits, (unsigned)a.n_tiles),
+                dim3((unsigned)a.n_kv_heads, (unsigned)a.splits.num_splits, (unsigned)a.n_tiles),
                 dim3(64 * kGroup * PARTS), 0, stream, a.tiles, a.positions, a.tables, a.max_pages,
-                a.pages_per_split, a.n_heads, a.n_kv_heads, a.num_splits,
+                a.splits.pages_per_split, a.n_heads, a.n_kv_heads, a.splits.num_splits,
                 reinterpret_cast<const f16*>(a.q), reinterpret_cast<const f16*>(a.k_pool),
                 reinterpret_cast<const f16*>(a.v_pool), reinterpret_cast<f16*>(a.out),
                 a.workspace, ml);
@@ -459,32 +455,18 @@ int tiles_launch(const PromptAttention& a, float2* ml, hipStream_t stream) {
 
 }  // namespace
 
-void prompt_splits(int n_tiles, int n_kv_heads, int span, int max_splits, int* num_splits,
-                   int* pages_per_split) {
-  constexpr int kStepPages = 2 * kKeys / kPage;
-  const long long blocks = (long long)n_tiles * n_kv_heads;
-  long long want = blocks > 0 ? kTargetBlocks / blocks : 1;
-  if (want > max_splits) want = max_splits;
-  if (want < 1) want = 1;
-  int pps = (int)((span + want - 1) / want);
-  if (pps < kMinSplitPages) pps = kMinSplitPages;
-  pps = (pps + kStepPages - 1) / kStepPages * kStepPages;
-  *pages_per_split = pps;
-  *num_splits = span > pps ? (span + pps - 1) / pps : 1;
-}
-
 int prompt_attention(const PromptAttention& a, hipStream_t stream) {
   if (a.n_tiles == 0) return LLMK_OK;
-  if (a.n_tiles > 65535 || a.num_splits > 65535) return LLMK_ERR_UNSUPPORTED;
-  float2* ml = reinterpret_cast<float2*>(a.workspace + (size_t)a.n_rows * a.num_splits *
+  if (a.n_tiles > 65535 || a.splits.num_splits > 65535) return LLMK_ERR_UNSUPPORTED;
+  float2* ml = reinterpret_cast<float2*>(a.workspace + (size_t)a.n_rows * a.splits.num_splits *
                                                             a.n_heads * kHeadDim);
-  const long long blocks = (long long)a.n_tiles * a.num_splits * a.n_kv_heads;
-  const int st = blocks <= kWideBlocks && a.pages_per_split * kPage > 2 * kKeys
+  const long long blocks = (long long)a.n_tiles * a.splits.num_splits * a.n_kv_heads;
+  const int st = blocks <= kWideBlocks && a.splits.pages_per_split * kPage > 2 * kKeys
                      ? tiles_launch<4>(a, ml, stream)
                      : tiles_launch<2>(a, ml, stream);
-  if (st != LLMK_OK || a.num_splits == 1) return st;
+  if (st != LLMK_OK || a.splits.num_splits == 1) return st;
   return merge_split_pieces(a.workspace, a.lens, a.out, a.n_rows, a.max_pages, a.n_heads,
-                            a.num_splits, a.pages_per_split, stream);
+                            a.splits.num_splits, a.splits.pages_per_split, stream);
 }
 
 }  // namespace llmk

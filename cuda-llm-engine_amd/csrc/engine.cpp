@@ -103,22 +103,23 @@ struct llmk_engine {
 
   // Pages the longest attention of the rows last set reads (position / 16 + 1).
   int rows_span = 0;
-  // The tiles of the rows last set, the pages the longest attention of their rows reads, and the
-  // rows in none.
-  int n_tiles = 0, tile_span = 0, loose_rows = 0;
+  // The tiles of the rows last set, the splits of their attention, and the rows in none.
+  int n_tiles = 0, loose_rows = 0;
+  llmk::PromptSplits tile_splits = {1, 1};
   long long tile_positions = 0;  // positions that the tiles' rows attend to, summed over the rows
   // Rows and logit rows uploaded by the last llmk_engine_set_rows: a pass may not ask for more,
   // since the device copies past them hold no checked indices.
   int rows_set = 0, logit_rows_set = 0;
 
-  // HIP graphs of the forward pass, keyed by (n_rows, n_logit_rows, resolved num_splits,
-  // host_argmax: whether the pass ends before the GPU argmax, n_tiles, tile_span and whether rows
-  // are left over, the last three 0 for a pass that takes no tiles)
+  // HIP graphs of the forward pass, keyed by (n_rows, n_logit_rows, resolved num_splits (0 where no
+  // row attends as a decode row), host_argmax: whether the pass ends before the GPU argmax, and the
+  // prompt tiles' launch: n_tiles and tile_splits, all 0 for a pass that takes no tiles)
   struct Graph {
     bool seen = false;
     hipGraphExec_t exec = nullptr;
   };
   std::map<std::tuple<int, int, int, int, int, int, int>, Graph> graphs;
+  int tiled_graphs = 0;  // the keys of passes that take tiles
   hipStream_t sched_stream = nullptr;  // the stream the scheduler callbacks run on
   bool fuse_rows = true;  // passes of <= LLMK_LINEAR_ROWS_MAX rows use the fused projections
   // LLMK_ENGINE_HOST_ARGMAX: the pass ends with the logits; the scheduler callbacks copy them
@@ -192,7 +193,7 @@ constexpr int kTileMinRows = 9;
 // Finds the runs of rows that continue one another: positions ascending by one, block tables
 // equal on every page the later row reads. Each run of at least kTileMinRows rows is cut into
 // tiles of kTileRows; fills tiles, row_lens and tile_lens and returns the tile count. The caller
-// has checked every position and table entry.
+// has checked every position and table entry. *span: pages that the longest attention in a tile reads.
 int find_tiles(int n, const int32_t* positions, const int32_t* tables, int max_pages,
                llmk::PromptTile* tiles, int32_t* row_lens, int32_t* tile_lens, int* span,
                int* loose, long long* attended) {
@@ -509,8 +510,10 @@ extern "C" int llmk_engine_set_rows(llmk_engine* e, int n_rows, const int32_t* t
   e->rows_span = span;
   if (n_logit_rows > 0) memcpy(h_logit, logit_rows, n_logit_rows * sizeof(int32_t));
   memcpy(h_tables, block_tables, (size_t)n_rows * P * sizeof(int32_t));
+  int tile_span = 0;
   e->n_tiles = find_tiles(n_rows, positions, block_tables, P, h_tiles, h_row_lens, h_tile_lens,
-                          &e->tile_span, &e->loose_rows, &e->tile_positions);
+                          &tile_span, &e->loose_rows, &e->tile_positions);
+  e->tile_splits = llmk::prompt_splits(e->n_tiles, e->cfg.n_kv_heads, tile_span, kMaxSplits);
   hipStream_t s = static_cast<hipStream_t>(stream);
   st = (int)hipMemcpyAsync(e->in_buf, e->staging, e->in_bytes, hipMemcpyHostToDevice, s);
   if (st == LLMK_OK) st = (int)hipEventRecord(e->staged, s);
@@ -593,8 +596,7 @@ static int attention(llmk_engine* e, int l, int n, bool tiled, int num_splits, v
   a.max_pages = e->max_pages;
   a.n_heads = m.n_heads;
   a.n_kv_heads = m.n_kv_heads;
-  llmk::prompt_splits(e->n_tiles, m.n_kv_heads, e->tile_span, kMaxSplits, &a.num_splits,
-                      &a.pages_per_split);
+  a.splits = e->tile_splits;
   return llmk::prompt_attention(a, static_cast<hipStream_t>(s));
 }
 
@@ -663,6 +665,7 @@ extern "C" int llmk_engine_set_option(llmk_engine* e, int option, int value) {
         for (auto& kv : e->graphs)
           if (kv.second.exec) (void)hipGraphExecDestroy(kv.second.exec);
         e->graphs.clear();
+        e->tiled_graphs = 0;
       }
       e->fuse_rows = value != 0;
       return LLMK_OK;
@@ -816,6 +819,10 @@ extern "C" int llmk_engine_reset_pools(llmk_engine* e, void* stream) {
                              static_cast<hipStream_t>(stream));
 }
 
+// Graphs kept of passes that take prompt tiles: a caller with ever other mixes of rows would fill
+// memory with them. Passes past that run eagerly.
+constexpr int kMaxTiledGraphs = 256;
+
 extern "C" int llmk_engine_forward_graph(llmk_engine* e, int n_rows, int n_logit_rows,
                                          int num_splits, void* stream) {
   if (!e || !stream) return LLMK_ERR_INVALID_VALUE;
@@ -829,9 +836,16 @@ extern "C" int llmk_engine_forward_graph(llmk_engine* e, int n_rows, int n_logit
   if (!rows_uploaded(e, n_rows, n_logit_rows)) return LLMK_ERR_INVALID_VALUE;
   num_splits = resolve_splits(e, n_rows, num_splits);  // the key holds the launch shapes
   const bool tiled = takes_tiles(e, n_rows, false);
-  llmk_engine::Graph& g = e->graphs[std::make_tuple(
-      n_rows, n_logit_rows < 0 ? -1 : n_logit_rows, num_splits, e->host_argmax ? 1 : 0,
-      tiled ? e->n_tiles : 0, tiled ? e->tile_span : 0, tiled && e->loose_rows > 0 ? 1 : 0)];
+  const auto key = std::make_tuple(
+      n_rows, n_logit_rows < 0 ? -1 : n_logit_rows, tiled && e->loose_rows == 0 ? 0 : num_splits,
+      e->host_argmax ? 1 : 0, tiled ? e->n_tiles : 0, tiled ? e->tile_splits.num_splits : 0,
+      tiled ? e->tile_splits.pages_per_split : 0);
+  if (tiled && e->graphs.find(key) == e->graphs.end()) {
+    if (e->tiled_graphs >= kMaxTiledGraphs)
+      return forward_pass(e, n_rows, n_logit_rows, num_splits, tiled, stream);
+    ++e->tiled_graphs;
+  }
+  llmk_engine::Graph& g = e->graphs[key];
   if (g.exec) return (int)hipGraphLaunch(g.exec, s);
   if (!g.seen) {  // first use: eager, which also makes the GEMM plans of these shapes
     g.seen = true;

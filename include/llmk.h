@@ -448,9 +448,10 @@ LLMK_API int llmk_engine_set_rows(llmk_engine* e, int n_rows, const int32_t* tok
  * max_pages; always capped at 32, the workspace. On a stream that is being captured the first
  * rule is skipped, so that a captured pass keeps enough splits for the longer contexts it may
  * be replayed with. Runs of 9 or more rows that continue one another (consecutive positions of
- * one sequence: a prompt) attend in tiles that share the K and V rows they read, when n_rows is
- * all the rows last set; not on a stream being captured, whose replays may hold other rows. Either
- * way gives the same values up to fp32 rounding. Allocates nothing; capturable into a HIP graph
+ * one sequence: a prompt) attend in tiles that share the K and V rows they read, with splits of
+ * their own whatever num_splits says, when n_rows is all the rows last set and the tiles are worth
+ * a launch beside the other rows'; not on a stream being captured, whose replays may hold other
+ * rows. Either way gives the same values up to fp32 rounding. Allocates nothing; capturable into a HIP graph
  * for a fixed n_rows.
  * ref: engine/batched.cu:107-120 (decode_step_gpu), :44-72 (layer_forward_batched), :150
  * (argmax_rows in model_decode_batch_greedy). */
@@ -490,11 +491,12 @@ LLMK_API int llmk_engine_set_option(llmk_engine* e, int option, int value);
 LLMK_API int llmk_engine_tune(llmk_engine* e, int n_rows, int n_logit_rows, void* stream);
 
 /* llmk_engine_forward through a HIP graph cache keyed by (n_rows, n_logit_rows, the resolved
- * split count -- num_splits <= 0 resolved against the rows last uploaded, as above -- and the
- * LLMK_ENGINE_HOST_ARGMAX setting):
+ * split count -- num_splits <= 0 resolved against the rows last uploaded, as above --, the
+ * LLMK_ENGINE_HOST_ARGMAX setting, and, where rows attend in tiles, the number of tiles and their
+ * splits, which a prompt's chunks mostly share):
  * the first call of a key runs eagerly (choosing the GEMM plans), the second captures the pass
- * on `stream` and instantiates it, later calls launch the instance. Same results as
- * llmk_engine_forward. `stream` must not be the null stream (it cannot be captured) and must
+ * on `stream` and instantiates it, later calls launch the instance; past 256 keys with tiles,
+ * passes of new ones run eagerly. Same results as llmk_engine_forward. `stream` must not be the null stream (it cannot be captured) and must
  * not be capturing already; the rows are whatever llmk_engine_set_rows uploaded last. */
 LLMK_API int llmk_engine_forward_graph(llmk_engine* e, int n_rows, int n_logit_rows,
                                        int num_splits, void* stream);

@@ -739,6 +739,33 @@ def test_prompt_tiles_replayed_with_other_rows(llmk):
         assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1]), rep
 
 
+def test_prompt_chunks_replayed_at_other_positions(llmk):
+    """A prompt's chunks through the engine's graph cache: from position 150 on they share a launch
+    shape, so the third of them is a replay whose splits end elsewhere than when it was captured.
+    Every chunk gives the bits of an eager pass."""
+    w = tiny_weights(0x5EED0280, embed_std=0.5)
+    rng = np.random.default_rng(0x5EED0281)
+    e = make_engine(llmk, TINY, w, 40, 24, 24)
+    s = torch.cuda.Stream()
+    n = 40
+    for start in (0, 60, 150, 170, 331, 150, 200, 344):
+        rows = (rng.integers(0, TINY["vocab"], n).astype(np.int32),
+                np.arange(start, start + n, dtype=np.int32),
+                np.array([rng.permutation(24).astype(np.int32)] * n))
+        fill = torch.from_numpy(rng.standard_normal(24 * 16 * 64).astype(np.float16))
+        out = []
+        for graph in (False, True):
+            for l in range(e.cfg.n_layers):
+                e.write_pool(llmk.BUF_K_POOL, l, fill)
+                e.write_pool(llmk.BUF_V_POOL, l, fill)
+            torch.cuda.synchronize()
+            e.set_rows(*rows, [n - 1], stream=s)
+            (e.forward_graph if graph else e.forward)(n, 1, stream=s)
+            torch.cuda.synchronize()
+            out.append((e.logits(1).view(torch.int16), e.residual(n).view(torch.int16)))
+        assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1]), start
+
+
 def test_engine_loads_the_reference_weight_format(llmk, tmp_path):
     weights = importlib.import_module("llmk.weights")
     w = tiny_weights(0x5EED0250, embed_std=0.5)
