@@ -570,6 +570,11 @@ static bool takes_tiles(const llmk_engine* e, int n, bool capturing) {
          (e->loose_rows == 0 || e->tile_positions >= kMixedMinPositions);
 }
 
+// The rows of a pass over n that attend as decode rows (at least 1): the split count is theirs.
+static int decode_rows(const llmk_engine* e, int n, bool tiled) {
+  return !tiled ? n : e->loose_rows > 0 ? e->loose_rows : 1;
+}
+
 // Attention of layer l over the pass's rows: prompt tiles share the K and V rows they read
 // (attention_prompt.hip); the other rows, or all of them without tiles, are decode rows. The
 // decode launch comes first: it writes NaN to rows of length 0, those in a tile.
@@ -795,8 +800,9 @@ extern "C" int llmk_engine_forward(llmk_engine* e, int n_rows, int n_logit_rows,
     if (st != LLMK_OK) return st;
     capturing = cap != hipStreamCaptureStatusNone;
   }
-  return forward_pass(e, n_rows, n_logit_rows, resolve_splits(e, n_rows, num_splits, capturing),
-                      takes_tiles(e, n_rows, capturing), stream);
+  const bool tiled = takes_tiles(e, n_rows, capturing);
+  num_splits = resolve_splits(e, decode_rows(e, n_rows, tiled), num_splits, capturing);
+  return forward_pass(e, n_rows, n_logit_rows, num_splits, tiled, stream);
 }
 
 extern "C" void* llmk_engine_buffer(llmk_engine* e, int which, int layer) {
@@ -834,8 +840,9 @@ extern "C" int llmk_engine_forward_graph(llmk_engine* e, int n_rows, int n_logit
   if (n_rows < 0 || n_rows > e->max_rows || n_logit_rows > n_rows) return LLMK_ERR_INVALID_VALUE;
   if (n_rows == 0) return LLMK_OK;
   if (!rows_uploaded(e, n_rows, n_logit_rows)) return LLMK_ERR_INVALID_VALUE;
-  num_splits = resolve_splits(e, n_rows, num_splits);  // the key holds the launch shapes
   const bool tiled = takes_tiles(e, n_rows, false);
+  // the key holds the launch shapes
+  num_splits = resolve_splits(e, decode_rows(e, n_rows, tiled), num_splits);
   const auto key = std::make_tuple(
       n_rows, n_logit_rows < 0 ? -1 : n_logit_rows, tiled && e->loose_rows == 0 ? 0 : num_splits,
       e->host_argmax ? 1 : 0, tiled ? e->n_tiles : 0, tiled ? e->tile_splits.num_splits : 0,

@@ -656,8 +656,14 @@ def run_both_ways(llmk, e, rows, logit_rows, fill):
 PROMPT_PASSES = [
     [(9, 0)], [(31, 0)], [(32, 1)], [(33, 0)], [(64, 15)], [(65, 16)], [(130, 100)],
     [(10, 250)],                             # few rows far into a sequence: split over positions
-    [(16, 5), (8, 40), (40, 0)],             # 8 rows are too few for a tile
-    [0, 77, (20, 30), 5, (45, 0), 130, 131],  # decode rows around and between the prompts
+    # Beside decode rows, tiles that attend to fewer than 81920 positions run as decode rows too (8
+    # rows are too few for a tile) ...
+    [(16, 5), (8, 40), (40, 0)],
+    [0, 77, (20, 30), 5, (45, 0), 130, 131],
+    # ... and from there on in tiles: before, between and after decode rows, two prompts, and tiles
+    # split over positions, whose pieces meet beside those of the decode rows
+    [0, 300, (420, 0), 77, (9, 5), 419],
+    [500, (100, 1000), 3, 1099, (8, 20)],
 ]
 
 
@@ -679,10 +685,13 @@ def test_prompt_tiles_match_decode_rows(llmk, parts, odd):
         v[0, 0] = 60000.0
         w[name] = v.view(w[name].dtype)
     rng = np.random.default_rng(0x5EED0261)
-    max_pages = 18
+    max_pages = 70
     tables = rng.permutation(len(parts) * max_pages).astype(np.int32).reshape(-1, max_pages)
     tok, pos, tab, last = [], [], [], []
     ends = []
+    prompts = [p for p in parts if isinstance(p, tuple) and p[0] >= 9]
+    tiles = (len(prompts) == len(parts)
+             or sum(n * start + n * (n + 1) // 2 for n, start in prompts) >= 81920)
     for t, part in zip(tables, parts):
         n, start = part if isinstance(part, tuple) else (1, part)
         pos += range(start, start + n)
@@ -710,6 +719,8 @@ def test_prompt_tiles_match_decode_rows(llmk, parts, odd):
             assert bool(fin.any()) or odd
         d = a[fin] - b[fin]
         assert d.norm() <= 2e-3 * max(float(b[fin].norm()), 1e-6), (name, float(d.norm()))
+        if name == "residual" and not odd and tiles and len(pos) >= 64:
+            assert not torch.equal(a, b), "no sum rounds the other way: were there tiles?"
     assert seen_nan == odd or len(pos) < 12
 
 
