@@ -221,22 +221,29 @@ for _name, (_res, _args) in _SIGS.items():
     _fn.argtypes = _args
 
 
+class _NoFastCalls:
+    """Stands for the native calls where none are built for this interpreter: no answer to any."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
 def _load_fast_calls():
     """The native calls beside libllmk.so (csrc/fast_calls.c). They answer a status, or None where
     the checks below have to decide."""
     import importlib.machinery
     import importlib.util
+    raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)  # torch without a GPU: none
     for suffix in importlib.machinery.EXTENSION_SUFFIXES:
         path = os.path.join(_HERE, "_fast_calls" + suffix)
-        if os.path.exists(path):
+        if os.path.exists(path) and raw_stream is not None:
             spec = importlib.util.spec_from_file_location("_fast_calls", path)
             mod = importlib.util.module_from_spec(spec)
             spec.loader.exec_module(mod)
             mod.setup(torch.Tensor, torch.float16, torch.int32, torch.float32,
-                      torch.cuda.current_device, torch._C._cuda_getCurrentRawStream)
+                      torch.cuda.current_device, raw_stream)
             return mod
-    raise ImportError(f"_fast_calls not found in {_HERE}: build it first (python -c "
-                      "'import __graft_entry__; __graft_entry__.build()')")
+    return _NoFastCalls()
 
 
 _fast = _load_fast_calls()

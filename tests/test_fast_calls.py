@@ -1,8 +1,14 @@
 """The native calls behind the Python face (csrc/fast_calls.c): they make the call when every
 argument is plainly right, and otherwise answer None with no exception set, so that the Python
-checks decide."""
+checks decide. They are optional, in the build and in the package."""
+import os
+import subprocess
+import sys
+
 import pytest
 import torch
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 DEV = "cuda:0"
 
@@ -35,6 +41,46 @@ def test_no_answer_for_anything_but_cuda_tensors(llmk, name):
     for i in range(len(args)):
         for bad in (None, "x", -1, 1 << 70, 1.5, object()):
             assert f(*args[:i], bad, *args[i + 1:]) is None
+
+
+def test_package_loads_without_the_native_calls(tmp_path):
+    pkg = os.path.join(ROOT, "cuda-llm-engine_amd")
+    for name in os.listdir(pkg):
+        if not name.startswith(("_fast_calls", "__pycache__")):
+            os.symlink(os.path.join(pkg, name), tmp_path / name)
+    code = f"""
+import importlib.util, sys, torch
+spec = importlib.util.spec_from_file_location(
+    "llmk", {str(tmp_path / "__init__.py")!r}, submodule_search_locations=[{str(tmp_path)!r}])
+llmk = sys.modules["llmk"] = importlib.util.module_from_spec(spec)
+spec.loader.exec_module(llmk)
+x = torch.zeros(32, dtype=torch.float16)
+try:
+    llmk.residual_add(x, x, x, 32)
+except llmk.LlmkError as e:
+    assert "must be a CUDA tensor" in str(e)
+    print("refused", llmk.version())
+"""
+    out = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True)
+    assert out.returncode == 0 and out.stdout.startswith("refused"), out.stderr
+
+
+def test_library_configures_without_python_headers(tmp_path):
+    out = subprocess.run(["cmake", "-S", ROOT, "-B", str(tmp_path), "-DLLMK_BUILD_TESTS=OFF",
+                          "-DCMAKE_DISABLE_FIND_PACKAGE_Python3=ON"],
+                         capture_output=True, text=True)
+    assert out.returncode == 0, out.stderr
+    assert "without the Python face's native calls" in out.stdout
+
+
+@pytest.mark.gpu
+def test_operators_without_the_native_calls(llmk, monkeypatch):
+    monkeypatch.setattr(llmk, "_fast", llmk._NoFastCalls())
+    x = torch.randn(4, 2048, device=DEV).half()
+    out = torch.empty_like(x)
+    llmk.residual_add(x, x, out, x.numel())
+    torch.cuda.synchronize()
+    assert torch.equal(out, x + x)
 
 
 @pytest.mark.gpu
