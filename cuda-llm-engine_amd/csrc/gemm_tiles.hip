@@ -24,12 +24,13 @@
 //   - the row tiles of one feature tile run on one XCD, next to each other: W crosses HBM once.
 // The product is W x^T (v_mfma_f32_16x16x32_f16, A: 16 features, B: 16 rows of x), so a lane ends
 // up with 4 consecutive features of one row. Same box, cold W, inside a graph, us, hipBLASLt's
-// first choice (tuned) -> here:
-//   in x out        40 rows              64 rows             128 rows            256 rows
-//   2048 x 3072     11.8 (8.7) -> 7.4    12.0 (8.9) -> 7.9   14.6 (10.7) -> 10.0  13.4 (13.5) -> 12.0
-//   2048 x 2048     11.3 (7.2) -> 7.0    11.7 (7.4) -> 7.4   11.2 (8.4) -> 7.5    12.0 (10.4) -> 9.6
-//   2048 x 16384    18.6 (18.2) -> 14.5  18.9 (18.4) -> 15.3 21.7 (21.8) -> 20.9  30.1 (30.3) -> 26.4
-//   8192 x 2048     14.5 (14.3) -> 12.8  22.8 (16.4) -> 13.8 21.7 (20.9) -> 16.1  27.9 (27.4) -> 21.5
+// first choice -> here (tuned, hipBLASLt takes 8.7, 7.2, 18.2 and 14.3 us at 40 rows, 13.5, 10.4,
+// 30.3 and 27.4 at 256):
+//   in x out        40 rows        64 rows        128 rows       256 rows
+//   2048 x 3072     8.9 -> 6.4     9.3 -> 6.5     12.2 -> 8.1    11.1 -> 11.0
+//   2048 x 2048     8.8 -> 6.4     9.2 -> 6.4     8.8 -> 6.6     10.1 -> 8.1
+//   2048 x 16384    18.0 -> 14.5   18.1 -> 15.4   22.1 -> 19.8   29.3 -> 26.8
+//   8192 x 2048     14.4 -> 12.7   22.6 -> 14.1   21.8 -> 16.4   27.6 -> 21.7
 #include "gemm_tiles.hpp"
 
 #include "layer_ops.hpp"
@@ -337,20 +338,23 @@ using T64x64 = Tile<2, 2, 2, 2, 2, 2, 3, 2>;
 using T64x128 = Tile<2, 2, 4, 2, 2, 2, 3, 4>;
 using T128x128 = Tile<4, 2, 2, 4, 1, 2, 4, 2>;
 constexpr int kTiles = 5;
-// What a launch takes by shape, in us: start + per_stage * (128-wide stages per CU - free), with
-// the blocks in rounds of one per CU. Fitted to sweeps of every shape and split count over 9 to 256
-// rows of 2048 x 3072, 2048, 16384 and 128256, 8192 x 2048, 4096 x 24576, 12288 x 4096, 1024 x
-// 8192 and 4096 x 1024; the choice it leads to is within 5% of the fastest in all but a few.
+// What a launch takes by shape, in us, with the blocks in rounds of one per CU and `n` stages of 128
+// to a block: start + (stage + full * the share of CUs with a block) * n, and round + round_stage *
+// n for each round after the first. Fitted to sweeps of every shape and split count over 9 to 512
+// rows of 22 matrices (2048 x 2048, 3072, 16384 and 32000, 8192 and 6144 x 2048, 1024 x 1024, 1536
+// and 8192, 4096 x 1024, 4096, 6144 and 24576, 12288 x 4096, 3072 x 3072, 4608 and 8192, 9216 x
+// 3072, 512 x 512, 640 x 4100, 256 x 16384, 16384 x 1024; cold W, in a graph) and tried on 18 more:
+// the choice it leads to takes 0.6% more than the fastest on average, 13% at most.
 struct Shape {
   int bm, bn;
-  float start, per_stage;
-  int free;  // stages that the launch's start hides
+  float start, stage, full, round, round_stage;
+  float piece;  // partial sums, per MB
 };
-constexpr Shape kShapes[kTiles] = {{32, 32, 4.5f, 0.25f, 3},
-                                   {64, 32, 4.5f, 0.43f, 5},
-                                   {64, 64, 4.4f, 0.64f, 0},
-                                   {128, 64, 5.0f, 0.80f, 0},
-                                   {128, 128, 4.5f, 1.25f, 0}};
+constexpr Shape kShapes[kTiles] = {{32, 32, 2.72f, 0.24f, 0.04f, 0.90f, 0.18f, 0.18f},
+                                   {64, 32, 3.28f, 0.25f, 0.10f, 1.77f, 0.31f, 0.20f},
+                                   {64, 64, 3.55f, 0.40f, 0.16f, 2.17f, 0.46f, 0.12f},
+                                   {128, 64, 4.57f, 0.57f, 0.24f, 2.95f, 0.72f, 0.14f},
+                                   {128, 128, 3.88f, 0.89f, 0.49f, 2.94f, 1.10f, 0.17f}};
 
 long long tile_blocks(const Shape& s, int T, int out) {
   return (long long)((T + s.bm - 1) / s.bm) * ((out + (long long)s.bn - 1) / s.bn);
@@ -390,37 +394,68 @@ int tiles_launch(int tile, const TileArgs& a, hipStream_t stream) {
 
 }  // namespace
 
-// Past 128 rows, products of more than one round of the largest tile stay with hipBLASLt, whose
-// larger tiles win there: 128256 outputs at 256 rows 181 us against 206 here, 4096 x 24576 at 160
-// rows 59 against 74 (at 128 rows 131 against 130 and 54 against 47). Past 256 rows so do short
-// products of more than one round of 64 x 64 tiles, unless a launch after them goes too: 2048 x
-// 3072 at 512 rows 15.3 against 16.2, where 2048 x 2048 takes 13.1 against 11.9, 8192 x 2048 37.0
-// against 29.6 and 12288 x 4096 83 against 68.
+// Where this library's tiles beat hipBLASLt's first choice; us, hipBLASLt / here. Up to 128 rows they
+// do, except past 24 rows of more than a round of 128 x 128 tiles if the product is short or, past
+// 32, its last round mostly empty: 1024 x 128256 at 16 rows 52.8 / 51.9, at 64 rows 59.1 / 64.7, 2048
+// x 40000 (1.2 rounds) at 32 rows 40.8 / 33.6, at 64 rows 43.0 / 46.2, 2048 x 128256 (3.9 rounds) 126
+// / 113. Past 128 rows hipBLASLt's larger tiles win:
+//   - more than a round of 128 x 128 tiles: 4096 x 24576 at 160 rows 54.6 / 83, 2048 x 32000 at 256
+//     43 / 53 (at most a round: 2048 x 16384 at 256 rows 30 / 27, 4096 x 8192 41 / 31);
+//   - 129 to 224 rows with more than a round of 64 x 64 tiles but no more than half a round of 128 x
+//     128 (less than half where in < 2048), unless a launch after them goes too: 4096 x 8192 at 129
+//     rows 25.7 / 27.9, 3072 x 8192 21.2 / 23.3, 4096 x 6144 at 200 rows 26.5 / 28.5 (at 160 rows
+//     28.1 / 26.6, at 256 40 / 28; 1024 x 8192 at 129 rows 12.8 / 10.9; past half a round: 2048 x
+//     12288 at 129 to 256 0.88 to 0.95 of it);
+//   - past 256 rows more than a round of 64 x 64 tiles, unless a launch goes too or the product is
+//     3 times as long as wide: 4096 x 6144 at 300 rows 30.7 / 38.7, 4096 x 4096 26.0 / 26.6, 2048 x
+//     6144 1.24 of it (6144 x 2048 0.75, 8192 x 2048 0.73, 9216 x 3072 0.90, 16384 x 4096 0.90; in one
+//     round 1024 x 1536 0.65, 2048 x 3072 0.99, 3072 x 3072 0.90).
 bool tiles_apply(const void* x, const void* w, const void* y, int T, int in, int out, bool fused) {
   if (T <= LLMK_LINEAR_ROWS_MAX || T > kTilesMaxRows || in % 128 != 0 || out % 4 != 0 ||
       !aligned16(x) || !aligned16(w) || (reinterpret_cast<uintptr_t>(y) & 7u) != 0)
     return false;
   const int cus = device_cus();
-  if (T > 128 && tile_blocks(kShapes[kTiles - 1], T, out) > cus) return false;
-  return T <= 256 || fused || in >= 4096 || tile_blocks(kShapes[2], T, out) <= cus;
+  const long long large = tile_blocks(kShapes[kTiles - 1], T, out);
+  if (T <= 128) {
+    const long long rounds = (large + cus - 1) / (cus > 0 ? cus : 1);
+    return large <= cus || T <= 24 ||
+           (in >= 2048 && (T <= 32 || 20 * large >= 17 * rounds * cus));
+  }
+  const bool one_round = tile_blocks(kShapes[2], T, out) <= cus;
+  if (large > cus) return false;
+  if (fused || one_round) return true;
+  if (T > 256) return in >= 3LL * out;
+  return T > 224 || 2 * large > cus || (in < 2048 && 2 * large == cus);
 }
 
-// The cheapest shape and split count by the model at kShapes. Splits add their partial sums, written
-// and read at 6 TB/s, and with reduce_launch a launch of 2.5 us.
+// The cheapest shape and split count by the model at kShapes; splits add their partial sums, to
+// k_tiles_reduce, with reduce_launch, or to the consumer's reads. The model does not know that wide
+// matrices past kWideW weights come from HBM alone. Their fastest shape stages the fewest bytes (128
+// x 128), or, if W takes more than a round of it, to 32 rows, multiplies the least (32 x 32): 2048 x
+// 128256 with 32 x 32 / 64 x 64 / 128 x 128 tiles at 16 rows 92 / 102 / 100 us, at 64 rows 150 / 117 /
+// 113; 4096 x 24576, one round, at 16 rows 37.0 / 43 / 40.8, at 64 rows 50 / 48 / 42.7.
+constexpr long long kWideW = 64 << 20;
+constexpr int kWideOut = 16384;
+
 TilePlan tiles_plan(int T, int in, int out, size_t max_floats, bool reduce_launch) {
   const int cus = device_cus() > 0 ? device_cus() : 256;
+  const bool rounds = tile_blocks(kShapes[kTiles - 1], T, out) > cus;
+  if ((long long)in * out >= kWideW && out >= kWideOut && (T > 24 || rounds))
+    return {T <= 32 && rounds ? 0 : kTiles - 1, 1};
   TilePlan best = {0, 1};
   float best_us = 0.0f;
   for (int tile = 0; tile < kTiles; ++tile) {
     const Shape& s = kShapes[tile];
-    const long long blocks = tile_blocks(s, T, out);
     for (int splits = 1; splits <= 8 && splits <= in / 128; splits *= 2) {
       const double floats = (double)splits * T * out;
       if (splits > 1 && floats > (double)max_floats) break;
-      const long long rounds = (blocks * splits + cus - 1) / cus;
-      const float stages = (float)rounds * (float)in / 128.0f / (float)splits - (float)s.free;
-      float us = s.start + s.per_stage * (stages > 0.0f ? stages : 0.0f);
-      if (splits > 1) us += (float)(floats * 8.0 / 6e6) + (reduce_launch ? 2.5f : 0.0f);
+      const long long blocks = tile_blocks(s, T, out) * splits;
+      const float n = (float)in / 128.0f / (float)splits, mb = (float)(floats * 4e-6);
+      const float more = (float)((blocks + cus - 1) / cus - 1);  // rounds after the first
+      const float share = blocks < cus ? (float)blocks / (float)cus : 1.0f;
+      float us = s.start + (s.stage + s.full * share) * n + more * (s.round + s.round_stage * n);
+      if (splits > 1)
+        us += s.piece * mb + (reduce_launch ? 1.4f + 0.18f * mb + 0.30f * (float)splits : 0.12f * mb);
       if ((tile == 0 && splits == 1) || us < best_us) {
         best = {tile, splits};
         best_us = us;

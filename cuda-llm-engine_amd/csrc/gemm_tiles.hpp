@@ -16,7 +16,7 @@ struct TilePlan {
 };
 
 // Whether y[T, out] = x[T, in] W^T runs here: 9 .. kTilesMaxRows rows, in a multiple of 128, out
-// of 4, x and w 16-byte and y 8-byte aligned, and not so large that hipBLASLt wins. `fused`: the
+// of 4, x and w 16-byte and y 8-byte aligned, and where hipBLASLt does not win. `fused`: the
 // product's consumer is part of the launch, or adds up its pieces itself.
 bool tiles_apply(const void* x, const void* w, const void* y, int T, int in, int out, bool fused);
 

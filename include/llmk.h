@@ -303,8 +303,8 @@ LLMK_API void llmk_blas_destroy(llmk_blas* h);
  * (a PyTorch Linear without bias); fp16 in and out, fp32 accumulation. With T <= 8,
  * in_features % 512 == 0 and x, W 16-byte aligned it runs llmk_linear_rows. With 9 to 512 rows,
  * in_features % 128 == 0, out_features % 4 == 0, x, W 16-byte and y 8-byte aligned it runs this
- * library's tiles (partial sums in the handle's workspace), except, past 128 rows, products so
- * large that hipBLASLt is faster. Otherwise the first call of a shape takes hipBLASLt's heuristic
+ * library's tiles (partial sums in the handle's workspace), except where hipBLASLt is faster
+ * (wide products, mostly past 128 rows). Otherwise the first call of a shape takes hipBLASLt's heuristic
  * choice (make that call outside graph capture) and later calls only enqueue. ref: kernels/linear.cuh:5-7, kernels/linear.cu:5-25 (linear;
  * cublasHandle_t -> llmk_blas*). */
 LLMK_API int llmk_linear(llmk_blas* h, const uint16_t* x, const uint16_t* w, uint16_t* y, int T,
