@@ -1,12 +1,13 @@
 """GPU parity of the decode-step pieces and the engine against the CPU oracle.
 
-- llmk_linear (hipBLASLt) vs the oracle's projection, with the reference's projection test rule
-  |d| <= 3e-3 + 8e-3 |e| (ref: tests/test_linear.cu:47) at the engine's shapes.
+- llmk_linear (this library's kernels and hipBLASLt) vs the oracle's projection, with the
+  reference's projection test rule |d| <= 3e-3 + 8e-3 |e| (ref: tests/test_linear.cu:47) at the
+  engine's shapes.
 - llmk_qkv_rope_scatter and llmk_swiglu_rows (the fused layouts) vs the oracle's separate
   operations on the same data: bit-exact, like the unfused kernels.
 - The engine (llmk_engine_*) vs oracle.engine_forward on a small Llama-3 shape and on the
   Llama-3.2-1B shape: mixed prefill and decode rows, shuffled pages, teacher-forced steps.
-  Library GEMMs sum in their own order, so the bar is the reference's for its engine against
+  GEMMs sum in their own order, so the bar is the reference's for its engine against
   Hugging Face: relative L2 of every logit row below 5e-3 (ref:
   tests/test_generate_batched.cu:53), the same greedy token wherever the oracle's top two are
   clearly apart, and the same set of written pool slots with every other slot still 0x7F7F.
@@ -76,7 +77,10 @@ TILE_CASES = [(9, 128, 4), (9, 256, 3072), (31, 1152, 36), (32, 128, 2056), (33,
               (64, 640, 4100), (65, 2048, 8196), (127, 384, 128), (128, 8192, 132),
               (129, 4096, 1028), (200, 2048, 16380), (255, 1152, 260), (256, 8192, 2052),
               (256, 256, 16384), (257, 256, 64), (384, 4096, 1028), (512, 8192, 132),
-              (513, 256, 64), (12, 192, 64), (40, 256, 66), (130, 128, 32772)]
+              (513, 256, 64), (12, 192, 64), (40, 256, 66), (130, 128, 32772),
+              # splits of every tile, and wide matrices: one round of the largest tile, and more
+              (9, 3072, 2052), (9, 2048, 36), (33, 6144, 2052), (33, 6144, 4100), (65, 6144, 3076),
+              (65, 3072, 8196), (65, 8192, 2052), (26, 4096, 16384), (20, 2048, 32772)]
 
 
 @pytest.mark.parametrize("T,K,N", TILE_CASES)
@@ -323,19 +327,32 @@ def test_linear_rows_fused_preconditions(llmk):
 
 
 def test_linear_after_tuning_matches_oracle(llmk, orc, blas):
-    """llmk_blas_tune swaps a shape's algorithm for the fastest timed candidate; the result
-    keeps the same bar."""
-    T, K, N = 256, 2048, 3072
+    """llmk_blas_tune swaps a shape's algorithm, here one in use, for the fastest timed candidate; the
+    result keeps the same bar. 600 rows are hipBLASLt's."""
+    T, K, N = 600, 2048, 3072
     rng = np.random.default_rng(0x5EED0205)
     x, w = normal_f16(rng, (T, K)), normal_f16(rng, (N, K), std=0.02)
     dx, dw = dev(x), dev(w)
-    y = torch.empty(T * N, dtype=torch.float16, device=DEV)
+    y = torch.full((T * N,), float("nan"), dtype=torch.float16, device=DEV)
+    llmk.linear(blas, dx, dw, y, T, K, N)
+    y.fill_(float("nan"))
     llmk.blas_tune(blas, dx, dw, y, T, K, N)
+    torch.cuda.synchronize()
+    assert not torch.isnan(y).any(), "no candidate ran"
     y.fill_(float("nan"))
     llmk.linear(blas, dx, dw, y, T, K, N)
     torch.cuda.synchronize()
     bad, exact = linear_rule(host(y), orc.linear(x, w, T, K, N, threads=16).ravel())
     assert bad == 0 and exact > 0.9
+
+
+@pytest.mark.parametrize("T,K,N", [(4, 2048, 3072), (256, 2048, 3072)])
+def test_tuning_does_nothing_for_this_librarys_kernels(llmk, blas, T, K, N):
+    x, w = (torch.zeros(s, dtype=torch.float16, device=DEV) for s in (T * K, N * K))
+    y = torch.full((T * N,), float("nan"), dtype=torch.float16, device=DEV)
+    llmk.blas_tune(blas, x, w, y, T, K, N)
+    torch.cuda.synchronize()
+    assert torch.isnan(y).all()
 
 
 def test_linear_rejects_bad_arguments(llmk, blas):
@@ -650,6 +667,85 @@ def run_both_ways(llmk, e, rows, logit_rows, fill):
         out.append((e.logits(nl), e.residual(n), e.pool(llmk.BUF_K_POOL, e.cfg.n_layers - 1),
                     e.pool(llmk.BUF_V_POOL, e.cfg.n_layers - 1)))
     return out
+
+
+# Hidden, KV heads and MLP width of one layer, and the rows of a pass: every tile for the QKV and
+# gate/up epilogues (gate/up 0, 2, 3, 4, 4 and none, QKV 0, 0, 1, 0, 2 and 3), 1 to 8 pieces into the
+# norm and rows of 1, 2 and 4 vectors per thread there, an MLP width not a multiple of 16.
+FUSED_PASSES = [(2048, 8, 8192, (9, 40, 65, 129, 256, 512)), (4096, 2, 4096, (9, 40, 130)),
+                (8192, 1, 2048, (33, 200)), (1024, 4, 1032, (70, 250, 512))]
+
+
+@pytest.mark.parametrize("hidden,n_kv,inter,n", [(h, k, i, n) for h, k, i, ns in FUSED_PASSES
+                                                 for n in ns])
+def test_fused_projections_give_the_bits_of_the_separate_launches(llmk, hidden, n_kv, inter, n):
+    """A layer's pass against RMSNorm, llmk_qkv_rope_scatter, attention, llmk_add_rmsnorm and
+    llmk_swiglu_rows on products that are exact in any order: the first norm gives signs, the QKV
+    weights are whole numbers of 1/64, and every row of the others has one element, 1 or 2. So the
+    pools are the separate launches' to the bit. The second norm adds its squares in another order:
+    one of its values in some thousands rounds the other way (2^-11), and with it a gate or an up
+    value, the activation (silu's slope is at most 1.1, so 2.1 times as far) and the residual."""
+    rng = np.random.default_rng(0x5EED0290 + hidden + n)
+    eps, pages, splits = 1e-15, 3, 4
+    qdim, kvdim = 256 * n_kv, 64 * n_kv
+    cfg = llmk.ModelConfig(n_layers=1, hidden=hidden, n_heads=4 * n_kv, n_kv_heads=n_kv,
+                           inter=inter, vocab=n, eps=eps)
+
+    def half(a):
+        return torch.from_numpy(np.ascontiguousarray(a, np.float32)).half().to(DEV)
+
+    def pick(rows, cols):
+        at = np.concatenate([rng.permutation(cols) for _ in range(-(-rows // cols))])[:rows]
+        scale = rng.choice([1.0, 2.0], rows)
+        w = np.zeros((rows, cols), np.float32)
+        w[np.arange(rows), at] = scale
+        at, scale = torch.from_numpy(at).to(DEV), half(scale)
+        return half(w), lambda x: (x[:, at] * scale).contiguous()
+
+    signs = rng.choice([-1.0, 1.0], (n, hidden))
+    embed = half(signs * 2.0 ** -14)
+    wqkv = rng.integers(-8, 9, (qdim + 2 * kvdim, hidden)) / 64
+    (wo, o), (wg, gate), (wu, up), (wd, down) = (pick(*s) for s in (
+        (hidden, qdim), (inter, hidden), (inter, hidden), (hidden, inter)))
+    mlp_norm = half(1 + 0.1 * rng.standard_normal(hidden))
+    ones = half(np.ones(hidden))
+    e = llmk.Engine(cfg, n, pages, n * pages)
+    e.set_weights(embed, ones, [dict(
+        attn_norm=ones, wq=half(wqkv[:qdim]), wk=half(wqkv[qdim:qdim + kvdim]),
+        wv=half(wqkv[qdim + kvdim:]), wo=wo, mlp_norm=mlp_norm, w_gate=wg, w_up=wu, w_down=wd)])
+    pools = [torch.from_numpy(rng.standard_normal(n * pages * 16 * kvdim).astype(np.float16)).to(DEV)
+             for _ in range(2)]
+    e.write_pool(llmk.BUF_K_POOL, 0, pools[0])
+    e.write_pool(llmk.BUF_V_POOL, 0, pools[1])
+    pos = rng.integers(0, pages * 16, n).astype(np.int32)
+    tables = rng.permutation(n * pages).astype(np.int32).reshape(n, pages)
+    print(f"fused pass hidden={hidden} inter={inter} rows={n}", flush=True)
+    e.set_rows(np.arange(n, dtype=np.int32), pos, tables, [n - 1])
+    e.forward(n, 1, splits)
+
+    qkv = (torch.from_numpy(signs).to(DEV) @ torch.from_numpy(wqkv).to(DEV).t()).half()
+    q = torch.empty(n * qdim, dtype=torch.float16, device=DEV)
+    inv = torch.tensor(llmk.compute_rope_inv_freq(64, 500000.0, 32.0, 1.0, 4.0, 8192.0),
+                       dtype=torch.float32, device=DEV)
+    llmk.qkv_rope_scatter(qkv, qdim + 2 * kvdim, q, *pools, dev_i32(tables), dev_i32(pos), inv, n,
+                          pages, 16, 4 * n_kv, n_kv, 64)
+    attn = torch.empty(n, qdim, dtype=torch.float16, device=DEV)
+    ws = torch.empty(llmk.attention_decode_fast_workspace_floats(n, 4 * n_kv, splits), device=DEV)
+    llmk.attention_decode_fast(q, *pools, dev_i32(tables), dev_i32(pos + 1), attn, ws, n, pages, 16,
+                               4 * n_kv, n_kv, 64, splits)
+    x, normed = embed.clone(), torch.empty_like(embed)
+    llmk.add_rmsnorm(x, o(attn), mlp_norm, normed, n, hidden, eps)
+    act = torch.empty(n, inter, dtype=torch.float16, device=DEV)
+    llmk.swiglu_rows(torch.cat([gate(normed), up(normed)], 1).contiguous(), act, n, inter)
+    step = down(act)
+    llmk.residual_add(x, step, x, n * hidden)
+    torch.cuda.synchronize()
+    for which, want in ((llmk.BUF_K_POOL, pools[0]), (llmk.BUF_V_POOL, pools[1])):
+        assert np.array_equal(host(e.pool(which, 0)).ravel(), host(want))
+    got, want = e.residual(n).double(), x.double().cpu()
+    off = (got - want).abs()
+    assert bool((off <= 2.0 ** -9 * step.double().cpu().abs() + 2.0 ** -10 * want.abs()).all())
+    assert float((off > 0).double().mean()) < 2e-3
 
 
 # (length, start) of each prompt and the position of each decode row, in the order of the rows

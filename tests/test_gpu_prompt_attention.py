@@ -85,15 +85,68 @@ class Rows:
     def check(self, llmk, what=""):
         got, k, v = self.run(llmk)
         ref, spread = self.expected(k, v)
-        bound = 2.0 ** -10 * np.abs(ref) + 2.0 ** -10 * X + 2.0 ** -17 * spread + 2.0 ** -24
-        worst = np.abs(got - ref) / bound
-        bad = ~(worst <= 1)
-        assert not bad.any(), (what, int(bad.sum()), np.argwhere(bad)[:4], got[bad][:4], ref[bad][:4])
+        assert_close(got, ref, spread, what)
+
+
+def assert_close(got, ref, spread, what):
+    bound = 2.0 ** -10 * np.abs(ref) + 2.0 ** -10 * X + 2.0 ** -17 * spread + 2.0 ** -24
+    bad = ~(np.abs(got - ref) <= bound)
+    assert not bad.any(), (what, int(bad.sum()), np.argwhere(bad)[:4], got[bad][:4], ref[bad][:4])
+
+
+def random_rows(n_kv, n, start, seed):
+    """Random queries, keys and values in binary fractions, the keys' part along the queries growing
+    over the positions, so that the running maximum keeps rising (by 14 log2 units in all)."""
+    r = Rows(n_kv, n, start, seed)
+    r.wq[:, 1:5, 0] = 1.0
+    r.wq[:, 33:63, 36:48] = r.rng.integers(-1, 2, (4 * n_kv, 30, 12)) / 4
+    r.wk[:, 33:63, 20:36] = r.rng.integers(-1, 2, (n_kv, 30, 16)) / 4
+    r.wv[:, :, 20:36] = r.rng.integers(-2, 3, (n_kv, 64, 16)) / 4
+    # columns 1 to 15 count up from -1 to 1 over the positions
+    level = (start + np.arange(n)) * 16 // (start + n)
+    r.signs[:, 1:16] = np.where(level[:, None] >= np.arange(1, 16), 1.0, -1.0)
+    r.wk[:, 1:5, 1:16] = 0.625
+    if start:
+        for rows, std in zip(r.cached, (0.75, 1.0)):
+            rows[:] = r.rng.standard_normal(rows.shape) * std
+        k = r.cached[0].reshape(start, n_kv, 64)
+        k[:, :, 1:5] = 0.625 * 2 * (np.arange(start) * 16 // (start + n) - 7.5)[:, None, None]
+    return r
+
+
+# (kv heads, rows, first position), and what they launch: 8 waves over one step of one split, of
+# several splits, and over 17 steps of one split (more than 512 blocks); 16 waves over four steps of
+# one split, the last for half of them, and over splits of a step and a half.
+EVERY_LAUNCH = [(1, 9, 0), (2, 70, 500), (3, 33, 700), (8, 2100, 0), (8, 1000, 0), (8, 1024, 1),
+                (2, 33, 9000)]
+
+
+@pytest.mark.parametrize("n_kv,n,start", EVERY_LAUNCH)
+def test_every_launch(llmk, n_kv, n, start):
+    random_rows(n_kv, n, start, seed=n + start).check(llmk, (n_kv, n, start))
+
+
+@pytest.mark.parametrize("n_kv,n,start,odd", [(1, 40, 0, 20), (8, 1000, 0, 300), (8, 2100, 0, 2000),
+                                              (2, 100, 500, 530)])
+def test_rows_before_a_value_that_is_not_finite(llmk, n_kv, n, start, odd):
+    """Position odd has an infinite value in one head: rows before it, in its tile and chunk as well,
+    are as ever, rows from it on are not finite (the MLP spreads it over the row)."""
+    r = random_rows(n_kv, n, start, seed=odd)
+    r.signs[:, 50] = -1.0
+    r.signs[odd - start, 50] = 1.0
+    r.wv[0, 3, 0] = r.wv[0, 3, 50] = 40000.0
+    got, k, v = r.run(llmk)
+    assert np.isinf(v[odd, 0, 3]) and np.isfinite(v[start:odd]).all()
+    ref, spread = r.expected(k, np.where(np.isfinite(v), v, 0.0))
+    before = slice(0, odd - start)
+    assert_close(got[before], ref[before], spread[before], odd)
+    assert not np.isfinite(got[odd - start:]).any()
 
 
 # (kv heads, rows, first position), and what they launch: 8 waves over one step; the same in three
-# splits; 16 waves over several steps of one split, the last with wave sets that have no positions.
-LAUNCHES = [(1, 40, 0), (1, 300, 0), (8, 1000, 0)]
+# splits; 16 waves over several steps of one split, the last with wave sets that have no positions; 8
+# waves over 17 steps.
+LAUNCHES = [(1, 40, 0), (1, 300, 0), (8, 1000, 0), (8, 2100, 0)]
 
 
 @pytest.mark.parametrize("n_kv,n,start", LAUNCHES)
