@@ -1493,7 +1493,7 @@ class Bench:
                 eng.write_pool(which, l, fill)
         del fill
         self.free()
-        eng.tune(n)     # time hipBLASLt's candidates for this batch's projection shapes
+        eng.tune(n)     # time hipBLASLt's candidates for the projections it runs of this batch
         eng.set_rows(tokens, pos, tables)
         eng.forward(n)  # eager once before capture
         torch.cuda.synchronize()
@@ -1512,7 +1512,8 @@ class Bench:
         nbytes = wl.bytes_decode_step(lens)
         path = ("fused few-rows projections (libllmk) with the norms, RoPE + scatter, SwiGLU and "
                 "residual adds inside them" if n <= llmk.LINEAR_ROWS_MAX else
-                "hipBLASLt projections + libllmk kernels")
+                "libllmk's projections with RoPE + scatter, SwiGLU and the residual norms inside "
+                "them, the lm head at hipBLASLt")
         e = kernel_entry(f"decode step 1B, {n} seqs (graph)", nbytes, t, None, {
             "tokens_per_s": round(n / t["mean_s"], 1), "seqs": int(n),
             "context_tokens": int(lens.sum()), "layers": cfg.n_layers,
@@ -1524,7 +1525,7 @@ class Bench:
         del graph
         self.free()
         self.kernels[f"decode_step_1b_{n}"] = e
-        if n > llmk.LINEAR_ROWS_MAX:  # the projections are hipBLASLt calls: time a C++ caller too
+        if n > llmk.LINEAR_ROWS_MAX:  # the lm head is a hipBLASLt call: time a C++ caller too
             c = self.decode_step_cpp(cfg, tokens, pos, tables, used, 128, nbytes,
                                      max(20, self.K // 4), max(5, self.W // 4))
             if c:

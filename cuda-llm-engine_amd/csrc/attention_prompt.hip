@@ -19,16 +19,17 @@
 // Weights stay 32-bit values: each enters the second product as hi + lo, two fp16 halves of
 // 2^15 p, which doubles that product's 8 instructions to 16 a chunk; the vector work of the
 // softmax (about 6 instructions and one exponential per score) is the larger part. Down to p =
-// 2^-20 of the row's maximum the halves are as near as the decode kernels' fp32
-// weights, whose exponents are rounded; below, where lo runs out of exponents, what they leave goes through the product once
-// more, 2^39 times as large, which serves to p = 2^-59. Only chunks that hold such a weight pay for
-// it: 1507 rows 33.0 -> 34.1 us for the search, 32.6 -> 59.7 where every chunk does (scores of
-// standard deviation 4). Sums that keep their own registers, or the scores, spill: 50 us.
-// The running maximum is rounded up to a whole number of log2 units: the offset 15 - m is
-// then exact, so the scale 2^15 costs nothing, and rescaling is rarer. That holds for scores below
-// kLargeScore; past it (finite, but far from a trained model's) the same reference is kept as m + f,
-// f the row's largest exponent after m is taken off, and the exponents are made in two steps, so
-// that a row's largest weight stays 2^15 however m rounds. The next step's K and V are in registers
+// 2^-20 of the row's maximum the halves are as near as the decode kernels' fp32 weights, whose
+// exponents are rounded; below, where lo runs out of exponents, what they leave goes through the
+// product once more, 2^39 times as large, which serves to p = 2^-59. Only chunks that hold such a
+// weight pay for it: 1507 rows 33.0 -> 34.1 us for finding none, 32.6 -> 59.7 where every chunk has
+// some (scores of standard deviation 4). With the scores kept for it, or sums of its own, the
+// registers run out: 50 us.
+// The running maximum is rounded up to a whole number of log2 units: the offset 15 - m is then
+// exact, so the scale 2^15 costs nothing, and rescaling is rarer. That holds for scores below
+// kLargeScore; past it (finite, but far from a trained model's) the reference is m + f, f the row's
+// largest exponent after m is taken off, and the exponents are made in two steps, so that a row's
+// largest weight stays 2^15 however m rounds. The next step's K and V are in registers
 // while this one is used. At 4000 rows staging alone (LDS writes, V transposed, two barriers) takes
 // 32 of the 156 us, the loads 15.
 #include <math.h>

@@ -428,8 +428,10 @@ bool tiles_apply(const void* x, const void* w, const void* y, int T, int in, int
   return T > 224 || 2 * large > cus || (in < 2048 && 2 * large == cus);
 }
 
-// The cheapest shape and split count by the model at kShapes; splits add their partial sums, to
-// k_tiles_reduce, with reduce_launch, or to the consumer's reads. The model does not know that wide
+// The cheapest shape and split count by the model at kShapes; pieces are read again, by
+// k_tiles_reduce, with reduce_launch, or by the consumer: the residual add and norm of 256 rows of
+// 2048 take 5.1 us over 1, 4 or 8 pieces, so what counts there is the launch before it (8192 x 2048 at
+// 256 rows: 128 x 128 in 8 pieces 17.8 us, 128 x 64 in 4 19.3). The model does not know that wide
 // matrices past kWideW weights come from HBM alone. Their fastest shape stages the fewest bytes (128
 // x 128), or, if W takes more than a round of it, to 32 rows, multiplies the least (32 x 32): 2048 x
 // 128256 with 32 x 32 / 64 x 64 / 128 x 128 tiles at 16 rows 92 / 102 / 100 us, at 64 rows 150 / 117 /
@@ -444,18 +446,22 @@ TilePlan tiles_plan(int T, int in, int out, size_t max_floats, bool reduce_launc
     return {T <= 32 && rounds ? 0 : kTiles - 1, 1};
   TilePlan best = {0, 1};
   float best_us = 0.0f;
+  const float per_cu = 1.0f / (float)cus;
+#pragma unroll
   for (int tile = 0; tile < kTiles; ++tile) {
     const Shape& s = kShapes[tile];
+    const float one = (float)tile_blocks(s, T, out) * per_cu;  // rounds of one split
     for (int splits = 1; splits <= 8 && splits <= in / 128; splits *= 2) {
-      const double floats = (double)splits * T * out;
-      if (splits > 1 && floats > (double)max_floats) break;
-      const long long blocks = tile_blocks(s, T, out) * splits;
-      const float n = (float)in / 128.0f / (float)splits, mb = (float)(floats * 4e-6);
-      const float more = (float)((blocks + cus - 1) / cus - 1);  // rounds after the first
-      const float share = blocks < cus ? (float)blocks / (float)cus : 1.0f;
+      const size_t floats = (size_t)splits * T * out;
+      if (splits > 1 && floats > max_floats) break;
+      const float mb = (float)floats * 4e-6f;
+      const float n = (float)in / 128.0f / (float)splits, rounds = one * (float)splits;
+      const float more = rounds > 1.0f ? __builtin_ceilf(rounds - 1e-3f) - 1.0f : 0.0f;
+      const float share = rounds < 1.0f ? rounds : 1.0f;
       float us = s.start + (s.stage + s.full * share) * n + more * (s.round + s.round_stage * n);
       if (splits > 1)
-        us += s.piece * mb + (reduce_launch ? 1.4f + 0.18f * mb + 0.30f * (float)splits : 0.12f * mb);
+        us += s.piece * mb + (reduce_launch ? 1.4f + 0.18f * mb + 0.30f * (float)splits
+                                            : 0.5f + 0.20f * (float)splits);
       if ((tile == 0 && splits == 1) || us < best_us) {
         best = {tile, splits};
         best_us = us;

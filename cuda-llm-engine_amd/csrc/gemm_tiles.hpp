@@ -34,7 +34,7 @@ int tiles_partial(const TilePlan& p, const uint16_t* x, const uint16_t* w, float
                   int in, int out, hipStream_t stream);
 
 // act[T, inter] = swiglu of the gate and up halves of fp16(x W^T), W [2 inter, in]; inter a
-// multiple of 16. The values of llmk_swiglu_rows.
+// multiple of 4. The values of llmk_swiglu_rows.
 int tiles_swiglu(const uint16_t* x, const uint16_t* w_gate_up, uint16_t* act, int T, int in,
                  int inter, hipStream_t stream);
 

@@ -283,12 +283,12 @@ LLMK_API int llmk_decode_nongemm_pass_layers(const llmk_decode_pass* pass, void*
 LLMK_API int llmk_decode_nongemm_pass_fused(const llmk_decode_pass* pass, void* stream);
 
 /* ------------------------------------------------------------------------------------------
- * The decode step around the kernels above: projections (hipBLASLt), the fused layouts they
+ * The decode step around the kernels above: projections, the fused layouts they
  * produce, and an engine that runs a whole Llama-3 forward pass over a batch of token rows.
  * ------------------------------------------------------------------------------------------ */
 
-/* A GEMM handle: one hipBLASLt handle, a 32 MiB workspace allocated at creation, and a cache
- * of per-shape plans. Calls on one handle share its workspace, so they must be ordered (one
+/* A GEMM handle: one hipBLASLt handle, a 32 MiB workspace allocated at creation (hipBLASLt's and
+ * this library's tiles'), and a cache of per-shape plans. Calls on one handle share its workspace, so they must be ordered (one
  * stream, or one handle per stream), as calls on one cuBLAS handle are. */
 typedef struct llmk_blas llmk_blas;
 LLMK_API int llmk_blas_create(llmk_blas** out);

@@ -2,7 +2,7 @@
 // C-ABI (llmk.h), with the reference engine's names where a concept maps one to one.
 //
 //  - linear(): ref: kernels/linear.cuh:5-7, with the cuBLAS handle replaced by a libllmk GEMM
-//    handle (llmk_blas*, hipBLASLt underneath).
+//    handle (llmk_blas*; this library's kernels up to 512 rows of most shapes, else hipBLASLt).
 //  - PageAllocator, Request, SchedulerStats, run_scheduler(): ref: engine/paging.h:7-23,
 //    engine/scheduler.h:6-27. The reference's scheduler takes (Model&, PagedKVCache&,
 //    BatchState&): here one llmk::Engine holds the weights, the pools and the batch buffers, so
